@@ -238,26 +238,245 @@ __global__ __launch_bounds__(kThreads) void evict_kernel(const half_t* __restric
 // next target row, each by a running fp32 sum over the vocabulary compared
 // against r (with its "tok == 0" update rule: a hit at index 0 is replaced by
 // the next hit).  The sampled indices depend on the exact fp32 value of every
-// partial sum, so each sum is accumulated serially in index order, as there.
-// Two workgroups of two waves per batch row: one computes Z and then the
-// residual sample, the other the bonus token, concurrently.  In each, wave 1
-// loads kChunk consecutive elements and stages their terms (differences, the
-// division by Z) into LDS -- for Z and the residual only the terms that change
-// the sum, compacted in index order with their indices -- while lane 0 of
-// wave 0 runs only the dependent adds of the previous chunk, 64 terms per
-// batch, and tests the running sum once per batch: sums only grow, so the
-// first hit lies in the batch where the test first passes, and lane 0 replays
-// that batch's adds one by one (the same adds in the same order, so the same
-// sums) to find it.  The sample and bonus scans stop at their first decisive
-// hit.  (Config 9: 327 us with one workgroup per row staging and adding in
-// turn, 240 with the compaction, 130 with staging and adds on separate waves.)
+// partial sum, i.e. on the rounding of each of the V serial additions.
+//
+// Those serial sums are computed in parallel, bit for bit.  While the running
+// sum s stays inside one binade it is n * g with g the ulp there and n an
+// integer, and adding a term t >= 0 moves n by an integer: rne(t / g), except
+// that an exact tie (t / g = k + 1/2) goes to the neighbour that makes n even.
+// A term is therefore a map from the parity of n to an increment, a pair
+// (d0, d1), and such pairs compose associatively: a wave scans the pairs of
+// its lanes' terms, a workgroup those of its waves.  A prefix is valid while
+// n <= 2^24; where it passes that (s leaves its binade), where a term is
+// negative or not finite, or where the comparison with r first holds, the
+// wave that owns the place walks it: it finds the first such lane by the same
+// scan, adds that lane's terms in fp32 one by one, and goes on from the sum it
+// gets.  A row of a thousand or more terms doubles its sum only a few times,
+// so nearly all of them go through the scans.
+//
+// Bound by the latency of those passes (about 1.5 us a tile of 8192 terms, a
+// few more per row for the binades), not by bytes: a row of 32000 is read at
+// the rate one CU can pull.  Two workgroups per row run concurrently: Z, then
+// the residual sample; the bonus token.  One lane adding all the terms in turn
+// from LDS, fed by a second wave, took 180 us for 16 rows of 32000 words
+// and K = 4; this takes 63 us.
 namespace spec {
 
-constexpr int kMaxK = 8;     // SPEC_MAX_K (flash_attn_kernel.cu:3851)
-constexpr int kChunk = 2048;  // elements per staged chunk (32 per lane)
-constexpr int kPerLane = kChunk / 64;
+constexpr int kMaxK = 8;      // SPEC_MAX_K (flash_attn_kernel.cu:3851)
+constexpr int kWaves = 16;
+constexpr int kSpecThreads = kWaves * 64;
+constexpr int kTerms = 8;     // consecutive terms per thread and tile
+constexpr int kTile = kSpecThreads * kTerms;
+constexpr uint32_t kTop = 1u << 24;  // n at the end of a binade
+constexpr uint32_t kCap = 1u << 25;  // increments saturate here (64 of them still fit 32 bits)
 
 enum ChainMode { kZ = 0, kResidual = 1, kPrefix = 2, kBonus = 3 };
+
+typedef float Terms __attribute__((ext_vector_type(kTerms)));
+typedef Terms Terms4 __attribute__((aligned(4)));  // rows start at any 4-byte boundary
+
+// Increment of n over a run of terms, for n even (d0) and odd (d1) before it.
+struct Inc {
+  uint32_t d0, d1;
+};
+__device__ __forceinline__ Inc then(const Inc& a, const Inc& b) {
+  Inc c;
+  c.d0 = min(a.d0 + ((a.d0 & 1u) ? b.d1 : b.d0), kCap);
+  c.d1 = min(a.d1 + ((a.d1 & 1u) ? b.d0 : b.d1), kCap);
+  return c;
+}
+__device__ __forceinline__ uint32_t advance(uint32_t n, const Inc& a) { return n + ((n & 1u) ? a.d1 : a.d0); }
+
+// x of the lane that DPP control CTRL names, 0 (no increment) where it names none
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp_from(uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, ROWS, 0xF, false));
+}
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ void scan_step(Inc& x) {
+  const Inc below = {dpp_from<CTRL, ROWS>(x.d0), dpp_from<CTRL, ROWS>(x.d1)};
+  x = then(below, x);
+}
+constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
+constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
+// Inclusive scan over each row of 16 lanes.
+__device__ __forceinline__ void scan_row(Inc& x) {
+  scan_step<kRowShr1>(x);
+  scan_step<kRowShr2>(x);
+  scan_step<kRowShr4>(x);
+  scan_step<kRowShr8>(x);
+}
+
+// The ulp grid of a sum s >= 0: s = n * 2^exp.
+struct Grid {
+  uint32_t n;
+  int exp;
+};
+__device__ __forceinline__ Grid grid_of(float s) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, s);
+  const uint32_t e = u >> 23;
+  return Grid{(u & 0x7fffffu) | (e ? 0x800000u : 0u), static_cast<int>(e ? e : 1u) - 150};
+}
+__device__ __forceinline__ float sum_of(uint32_t n, int exp) {
+  return __builtin_amdgcn_ldexpf(static_cast<float>(n), exp);
+}
+// sums the scans apply to: not negative, not infinite, not NaN
+__device__ __forceinline__ bool on_grid(float s) { return s >= 0.0f && s < INFINITY; }
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+
+// t / g, exact up to the cap (0 for a negative t, which is never taken from here)
+__device__ __forceinline__ float terms_on(float t, int exp) {
+  return __builtin_amdgcn_fmed3f(__builtin_amdgcn_ldexpf(t, -exp), 0.0f, static_cast<float>(kCap));
+}
+
+// Inclusive scan of the wave's terms on the grid 2^exp; lanes that are not
+// `active` contribute nothing.
+__device__ __forceinline__ Inc scan_terms(const Terms& t, bool active, int exp) {
+  uint32_t sum = 0;
+  bool tie = false;
+#pragma unroll
+  for (int e = 0; e < kTerms; ++e) {
+    const float x = terms_on(t[e], exp);
+    const float q = __builtin_rintf(x);
+    tie |= fabsf(x - q) == 0.5f;
+    sum += static_cast<uint32_t>(q);
+  }
+  sum = active ? min(sum, kCap) : 0u;
+  if (__builtin_amdgcn_ballot_w64(tie && active) == 0) {
+    // no tie in the wave: plain increments (64 * 2^25 at most)
+    sum += dpp_from<kRowShr1>(sum);
+    sum += dpp_from<kRowShr2>(sum);
+    sum += dpp_from<kRowShr4>(sum);
+    sum += dpp_from<kRowShr8>(sum);
+    sum += dpp_from<kRowBcast15, 0xA>(sum);
+    sum += dpp_from<kRowBcast31, 0xC>(sum);
+    sum = min(sum, kCap);
+    return Inc{sum, sum};
+  }
+  Inc x = {0u, 0u};
+  if (active) {
+#pragma unroll
+    for (int e = 0; e < kTerms; ++e) {
+      const float v = terms_on(t[e], exp);
+      const float q = __builtin_rintf(v);
+      // a tie's even neighbour is q, its odd one the other
+      const uint32_t even = static_cast<uint32_t>(q);
+      const uint32_t odd = fabsf(v - q) == 0.5f ? 2u * static_cast<uint32_t>(v) + 1u - even : even;
+      x = then(x, Inc{even, odd});
+    }
+  }
+  scan_row(x);
+  scan_step<kRowBcast15, 0xA>(x);
+  scan_step<kRowBcast31, 0xC>(x);
+  return x;
+}
+
+// Where a chain stands: the running sum and what it has found.  Uniform over
+// the workgroup.
+struct Walk {
+  float s;
+  int tok;        // token found, valid with done
+  int zero_hit;   // a hit at index 0 was seen, the next hit decides
+  int done;
+};
+
+// In kZ and kResidual a term that does not contribute (target <= draft, or
+// past V) is -0.0, which leaves the sum unchanged and is never a hit; one that
+// does has its sign bit clear.  Past V every mode has -0.0.
+template <int MODE>
+__device__ __forceinline__ bool contributes(float t, int v, int V) {
+  if constexpr (MODE == kResidual) return !__builtin_signbit(t);
+  return v < V;
+}
+template <int MODE>
+__device__ __forceinline__ bool is_hit(float s, float r) {
+  if constexpr (MODE == kZ) return false;
+  if constexpr (MODE == kBonus) return s >= r;
+  return r < s;
+}
+
+// One wave takes its own 64 * kTerms terms (lane l: indices v0 .. v0 + kTerms)
+// from w to the end of them or to the token.
+template <int MODE>
+__device__ void walk_wave(const Terms& t, int v0, int V, float r, bool bad, bool contrib, Walk& w) {
+  const int lane = threadIdx.x & 63;
+  for (int from = 0; from < 64;) {
+    int at = from;
+    float s0 = w.s;
+    if (on_grid(w.s)) {
+      const Grid g = grid_of(w.s);
+      const Inc x = scan_terms(t, lane >= from, g.exp);
+      const uint32_t n = advance(g.n, x);
+      const float s = sum_of(n, g.exp);
+      const bool stop = lane >= from && (n > kTop || bad || (contrib && is_hit<MODE>(s, r)));
+      const uint64_t stops = __builtin_amdgcn_ballot_w64(stop);
+      if (stops == 0) {
+        w.s = lane_value(s, 63);
+        return;
+      }
+      at = __builtin_ctzll(stops);
+      if (at > from) s0 = lane_value(s, at - 1);
+    } else if (w.s != w.s) {
+      return;  // NaN from here on: no comparison holds
+    }
+    // lane `at` adds its terms one by one (every lane does, its own are kept)
+    float s = s0;
+    int tok = -1, zero_hit = w.zero_hit;
+#pragma unroll
+    for (int e = 0; e < kTerms; ++e) {
+      s += t[e];
+      const int v = v0 + e;
+      if (tok < 0 && contributes<MODE>(t[e], v, V) && is_hit<MODE>(s, r)) {
+        if (v == 0) zero_hit = 1;
+        else tok = v;
+      }
+    }
+    w.s = lane_value(s, at);
+    w.zero_hit = __builtin_amdgcn_readlane(zero_hit, at);
+    tok = __builtin_amdgcn_readlane(tok, at);
+    if (tok >= 0) {
+      w.tok = tok;
+      w.done = 1;
+      return;
+    }
+    from = at + 1;
+  }
+}
+
+struct Shared {
+  uint32_t d0[2][kWaves], d1[2][kWaves];  // increments of each wave's terms, by pass parity
+  int flags[2][kWaves];                   // 1: has a contributing term, 2: has one off the grid
+  Walk w;
+};
+
+// row[v0 .. v0 + kTerms), 0 past V
+__device__ __forceinline__ Terms load_terms(const float* row, int v0, int V) {
+  Terms x;
+  if (v0 + kTerms <= V) return *reinterpret_cast<const Terms4*>(row + v0);
+#pragma unroll
+  for (int e = 0; e < kTerms; ++e) x[e] = v0 + e < V ? row[v0 + e] : 0.0f;
+  return x;
+}
+
+// The chain's terms from row values a (and b).
+template <int MODE>
+__device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, float Z, int v0, int V) {
+  Terms t;
+#pragma unroll
+  for (int e = 0; e < kTerms; ++e) {
+    if constexpr (MODE == kZ || MODE == kResidual) {
+      const float d = a[e] - b[e];
+      t[e] = d > 0.0f && v0 + e < V ? (MODE == kZ ? d : d / Z) : -0.0f;
+    } else {
+      t[e] = v0 + e < V ? a[e] : -0.0f;
+    }
+  }
+  return t;
+}
 
 // Serial scan of row a (minus row b for kZ / kResidual) over [0, V).
 //  kZ:        *sum = the sum of the positive (a - b) in index order.
@@ -265,180 +484,90 @@ enum ChainMode { kZ = 0, kResidual = 1, kPrefix = 2, kBonus = 3 };
 //  kPrefix:   cs += a; hit when r < cs.
 //  kBonus:    cs += a; hit when cs >= r.
 // Returns the reference's token: the first hit, or the next hit if the first
-// is index 0 (0 without hits).  A term that does not contribute (a - b <= 0
-// for kZ / kResidual, or past V) is -0.0, which leaves a non-negative running
-// sum unchanged; a contributing term has its sign bit clear (+0.0 if the
-// division underflows), so the replay reads "contributed" off the sign.  For
-// kResidual the first v with r < cs always contributed (cs only grows where
-// a term is added); a later hit must contribute too.
-//
-// Two waves: wave 1 stages the terms of chunk c + 1 into one LDS buffer
-// while lane 0 of wave 0 adds chunk c from the other; one workgroup barrier
-// per chunk hands the buffers over.  kZ and kResidual stage only the
-// contributing terms, compacted in index order with their indices: adding a
-// non-contributing -0.0 to the non-negative running sum changes nothing, so
-// lane 0 runs the same adds in the same order over about half the terms for
-// unrelated target and draft rows.  Every wave runs the same number of
-// barriers: the loop is bounded by the chunk count and its early exit is read
-// from LDS after a barrier.
-struct Stage {
-  float t[2][kChunk + 64];  // terms (+ one batch of -0.0 padding)
-  int idx[2][kChunk];       // their indices (compacted modes)
-  int n[2];                 // terms staged
-  int done, tok;
-  float sum;
-};
-
+// is index 0 (0 without hits).  Every wave takes the same path through the
+// barriers: what decides it is read from LDS after one.
 template <int MODE>
 __device__ int chain(const float* __restrict__ a, const float* __restrict__ b, int V, float Z, float r, float* sum,
-                     Stage& st) {
-  constexpr bool kCompact = MODE == kZ || MODE == kResidual;
+                     Shared& sh) {
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int nchunks = (V + kChunk - 1) / kChunk;
-  // lane l holds elements c0 + 256 q + 4 l + e (q < kPerLane / 4, e < 4):
-  // 16-byte loads where the row allows them (V % 4 == 0 and 16-byte aligned
-  // rows), element loads otherwise
-  const bool vec = (V & 3) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0 &&
-                   (MODE == kPrefix || MODE == kBonus || (reinterpret_cast<uintptr_t>(b) & 15) == 0);
-  auto load = [&](int c0, float4_t (&x)[kPerLane / 4], float4_t (&y)[kPerLane / 4]) {
-#pragma unroll
-    for (int q = 0; q < kPerLane / 4; ++q) {
-      const int v0 = c0 + 256 * q + 4 * lane;
-      if (vec) {
-        const bool in = v0 < V;
-        x[q] = in ? *reinterpret_cast<const float4_t*>(a + v0) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (MODE == kZ || MODE == kResidual)
-          y[q] = in ? *reinterpret_cast<const float4_t*>(b + v0) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[q][e] = v0 + e < V ? a[v0 + e] : 0.0f;
-          if constexpr (MODE == kZ || MODE == kResidual) y[q][e] = v0 + e < V ? b[v0 + e] : 0.0f;
-        }
-      }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tid = threadIdx.x;
+  Walk w = {0.0f, 0, 0, 0};
+  constexpr bool kDiff = MODE == kZ || MODE == kResidual;
+  Terms xa = load_terms(a, tid * kTerms, V);
+  Terms xb = kDiff ? load_terms(b, tid * kTerms, V) : Terms(0.0f);
+  int pass = 0;
+  for (int c0 = 0; c0 < V && !w.done; c0 += kTile) {
+    const int v0 = c0 + tid * kTerms;
+    const Terms t = make_terms<MODE>(xa, xb, Z, v0, V);
+    if (c0 + kTile < V) {  // the next tile's values travel while this one is summed
+      xa = load_terms(a, v0 + kTile, V);
+      if constexpr (kDiff) xb = load_terms(b, v0 + kTile, V);
     }
-  };
-  // wave 1: stage chunk c into buffer c & 1
-  auto stage = [&](int c) {
-    const int c0 = c * kChunk;
-    const int buf = c & 1;
-    float4_t x[kPerLane / 4], y[kPerLane / 4];
-    load(c0, x, y);
-    float* t_out = st.t[buf];
-    if constexpr (kCompact) {
-      int base = 0;
+    bool bad = false, contrib = false;
 #pragma unroll
-      for (int q = 0; q < kPerLane / 4; ++q) {
-        float t[4];
-        bool f[4];
-        int below = 0, total = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float d = x[q][e] - y[q][e];
-          f[e] = d > 0.0f && c0 + 256 * q + 4 * lane + e < V;
-          t[e] = MODE == kZ ? d : d / Z;
-          const uint64_t bal = __builtin_amdgcn_ballot_w64(f[e]);
-          below += __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bal >> 32),
-                                             __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal), 0u));
-          total += __builtin_popcountll(bal);
-        }
-        // element order c0 + 256 q + 4 lane + e: lanes below first, then e
-        int pos = base + below;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (f[e]) {
-            t_out[pos] = t[e];
-            st.idx[buf][pos] = c0 + 256 * q + 4 * lane + e;
-            ++pos;
-          }
-        base += total;
-      }
-      t_out[base + lane] = -0.0f;  // pad the last batch of 64: no change, never a hit
-      if (lane == 0) st.n[buf] = base;
-    } else {
-#pragma unroll
-      for (int q = 0; q < kPerLane / 4; ++q) {
-        float4_t t4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) t4[e] = c0 + 256 * q + 4 * lane + e < V ? x[q][e] : -0.0f;  // past V: never a hit
-        *reinterpret_cast<float4_t*>(t_out + 256 * q + 4 * lane) = t4;
-      }
-      if (lane == 0) st.n[buf] = min(kChunk, V - c0);
+    for (int e = 0; e < kTerms; ++e) {
+      bad |= !(t[e] >= 0.0f && t[e] < INFINITY);
+      contrib |= contributes<MODE>(t[e], v0 + e, V);
     }
-  };
-
-  if (threadIdx.x == 0) st.done = 0;
-  if (wave == 1) stage(0);
-  __syncthreads();
-  float cs = 0.0f;        // lane 0 of wave 0: the running sum
-  int tok = 0;            // lane 0 of wave 0: the token found so far
-  bool zero_hit = false;  // lane 0 of wave 0: a hit at index 0 was seen, the next hit decides
-  for (int c = 0; c < nchunks; ++c) {
-    const int buf = c & 1;
-    if (wave == 1) {
-      if (c + 1 < nchunks) stage(c + 1);
-    } else if (lane == 0) {
-      const float* tb = st.t[buf];
-      const int n = st.n[buf];
-      bool done = false;
-      for (int h = 0; h < n && !done; h += 64) {
-        float4_t q[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) q[j] = *reinterpret_cast<const float4_t*>(tb + h + 4 * j);
-        const float cs0 = cs;
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) cs += q[j][e];
-        if constexpr (MODE != kZ) {
-          const bool crossed = (MODE == kBonus) ? (cs >= r) : (r < cs);
-          if (crossed || zero_hit) {
-            // replay the batch: the first hit, or the next one after a hit at 0
-            float x = cs0;
-            for (int k = 0; k < 64 && !done; ++k) {
-              if (h + k >= n) break;
-              const float t = tb[h + k];
-              x += t;
-              const bool contrib = MODE != kResidual || !__builtin_signbit(t);
-              const bool hit = (MODE == kBonus) ? (x >= r) : (r < x) && contrib;
-              if (!hit) continue;
-              const int v = kCompact ? st.idx[buf][h + k] : c * kChunk + h + k;
-              if (v == 0 && !zero_hit) {
-                zero_hit = true;
-              } else {
-                tok = v;
-                done = true;
-              }
-            }
-          }
+    const int flags = (__builtin_amdgcn_ballot_w64(contrib) ? 1 : 0) | (__builtin_amdgcn_ballot_w64(bad) ? 2 : 0);
+    const int waves = min(kWaves, (V - c0 + 64 * kTerms - 1) / (64 * kTerms));  // waves with terms
+    int from = 0;         // first wave whose terms are still to be added
+    bool direct = c0 == 0;  // walk the next wave without a pass: the sum starts at 0 and doubles often
+    while (from < waves) {
+      int at = from;
+      if (!direct && on_grid(w.s)) {
+        const Grid g = grid_of(w.s);
+        const int buf = pass & 1;
+        ++pass;
+        Inc x = {0u, 0u};
+        if (wave >= from) x = scan_terms(t, true, g.exp);
+        if (lane == 63) {
+          sh.d0[buf][wave] = x.d0;
+          sh.d1[buf][wave] = x.d1;
+          sh.flags[buf][wave] = flags;
         }
+        __syncthreads();
+        // lane l of each row of 16: wave l's end
+        Inc y = {sh.d0[buf][lane & 15], sh.d1[buf][lane & 15]};
+        const int f = sh.flags[buf][lane & 15];
+        scan_row(y);
+        const uint32_t n = advance(g.n, y);
+        const float s = sum_of(n, g.exp);
+        const bool stop = lane >= from && lane < waves &&
+                          (n > kTop || (f & 2) || ((f & 1) && is_hit<MODE>(s, r)));
+        const uint64_t stops = __builtin_amdgcn_ballot_w64(stop);
+        at = stops ? __builtin_ctzll(stops) : waves;
+        if (at > from) w.s = lane_value(s, at - 1);
+        if (at == waves) break;
+      } else if (!direct) {
+        __syncthreads();  // every wave has read sh.w
       }
-      if (done) st.done = 1;
+      direct = false;
+      if (wave == at) {
+        walk_wave<MODE>(t, v0, V, r, bad, contrib, w);
+        if (lane == 0) sh.w = w;
+      }
+      __syncthreads();
+      w = sh.w;
+      if (w.done || w.s != w.s) break;
+      from = at + 1;
     }
-    __syncthreads();  // chunk c consumed, chunk c + 1 staged
-    if (st.done) break;
+    if (w.s != w.s) break;
   }
-  if (threadIdx.x == 0) {
-    st.tok = tok;
-    st.sum = cs;
-  }
-  __syncthreads();
-  const int result = st.tok;
-  if (sum) *sum = st.sum;
-  __syncthreads();  // every thread has read tok / sum before the next chain resets them
-  return result;
+  __syncthreads();  // every wave has read sh.w and the last pass before the next chain writes them
+  if (sum) *sum = w.s;
+  return w.done ? w.tok : 0;
 }
 
 // Grid (B, 2): workgroup (b, 0) settles the acceptance steps of row b and,
 // after a rejection, samples the residual (Z, then the residual scan);
-// workgroup (b, 1) draws the bonus token.  Both run the (cheap) acceptance
-// steps themselves.
-__global__ __launch_bounds__(128) void verify_kernel(const float* __restrict__ target, const float* __restrict__ draft,
-                                                     const int64_t* __restrict__ draft_tokens,
-                                                     const float* __restrict__ rand, int32_t* __restrict__ accepted,
-                                                     int64_t* __restrict__ out, int K, int V) {
-  __shared__ __attribute__((aligned(16))) Stage st;
+// workgroup (b, 1) draws the bonus token.  Both run the acceptance steps
+// themselves, lane i step i.
+__global__ __launch_bounds__(kSpecThreads) void verify_kernel(
+    const float* __restrict__ target, const float* __restrict__ draft, const int64_t* __restrict__ draft_tokens,
+    const float* __restrict__ rand, int32_t* __restrict__ accepted, int64_t* __restrict__ out, int K, int V) {
+  __shared__ Shared sh;
   const int b = blockIdx.x;
   const int role = blockIdx.y;
   const float* tb = target + static_cast<size_t>(b) * (K + 1) * V;
@@ -447,44 +576,39 @@ __global__ __launch_bounds__(128) void verify_kernel(const float* __restrict__ t
   const float* rb = rand + static_cast<size_t>(b) * K;
   int64_t* ob = out + static_cast<size_t>(b) * (K + 1);
 
-  // acceptance steps (uniform: every thread reads the same values)
-  int acc = 0;
-  int rej = -1;
-  for (int i = 0; i < K; ++i) {
-    const int64_t t = tok_b[i];
-    const bool in_range = t >= 0 && t < V;
-    const float p = in_range ? tb[static_cast<size_t>(i) * V + t] : 0.0f;
-    const float q = in_range ? db[static_cast<size_t>(i) * V + t] : 0.0f;
-    const float accept_prob = fminf(1.0f, p / (q + 1e-10f));
-    if (rb[i] < accept_prob) {
-      ++acc;
-    } else {
-      rej = i;
-      break;
-    }
+  const int step = threadIdx.x & 63;
+  int64_t tok = 0;
+  bool rejects = false;
+  if (step < K) {
+    tok = tok_b[step];
+    const float r = rb[step];
+    const bool in_range = tok >= 0 && tok < V;
+    const float p = in_range ? tb[static_cast<size_t>(step) * V + tok] : 0.0f;
+    const float q = in_range ? db[static_cast<size_t>(step) * V + tok] : 0.0f;
+    rejects = !(r < fminf(1.0f, p / (q + 1e-10f)));
   }
+  const uint64_t rejections = __builtin_amdgcn_ballot_w64(rejects);
+  const int rej = rejections ? __builtin_ctzll(rejections) : -1;
+  const int acc = rej >= 0 ? rej : K;
   if (role == 0) {
-    if (threadIdx.x == 0) {
-      // every position is written: accepted tokens, then (after a rejection at
-      // rej) the sample at rej, the bonus at rej + 1 (workgroup (b, 1)) and -1 beyond
-      for (int i = 0; i < acc; ++i) ob[i] = tok_b[i];
-      if (rej >= 0)
-        for (int j = rej + 2; j <= K; ++j) ob[j] = -1;
-      accepted[b] = acc;
-    }
+    // every position is written: accepted tokens, then (after a rejection at
+    // rej) the sample at rej, the bonus at rej + 1 (workgroup (b, 1)) and -1 beyond
+    if (threadIdx.x < acc) ob[step] = tok;
+    if (rej >= 0 && static_cast<int>(threadIdx.x) >= rej + 2 && static_cast<int>(threadIdx.x) <= K) ob[threadIdx.x] = -1;
+    if (threadIdx.x == 0) accepted[b] = acc;
     if (rej >= 0) {
       const float* ti = tb + static_cast<size_t>(rej) * V;
       const float* di = db + static_cast<size_t>(rej) * V;
       float Z;
-      chain<kZ>(ti, di, V, 0.0f, 0.0f, &Z, st);
-      const int s = Z > 0.0f ? chain<kResidual>(ti, di, V, Z, rb[rej], nullptr, st)
-                             : chain<kPrefix>(ti, nullptr, V, 0.0f, rb[rej], nullptr, st);
+      chain<kZ>(ti, di, V, 0.0f, 0.0f, &Z, sh);
+      const int s = Z > 0.0f ? chain<kResidual>(ti, di, V, Z, rb[rej], nullptr, sh)
+                             : chain<kPrefix>(ti, nullptr, V, 0.0f, rb[rej], nullptr, sh);
       if (threadIdx.x == 0) ob[rej] = s;
     }
   } else {
     const int row = rej >= 0 ? rej + 1 : K;
     const float r = rb[rej >= 0 ? min(rej, K - 1) : K - 1];
-    const int bonus = chain<kBonus>(tb + static_cast<size_t>(row) * V, nullptr, V, 0.0f, r, nullptr, st);
+    const int bonus = chain<kBonus>(tb + static_cast<size_t>(row) * V, nullptr, V, 0.0f, r, nullptr, sh);
     if (threadIdx.x == 0) ob[row] = bonus;
   }
 }
@@ -531,7 +655,7 @@ extern "C" int fa_speculative_verify(const float* target_probs, const float* dra
   if (B == 0) return FA_OK;
   if (!target_probs || !draft_probs || !draft_tokens || !random_vals || !accepted_count || !output_tokens)
     return set_error(FA_ERR_INVALID_ARG, "%s: null pointer", fn);
-  hipLaunchKernelGGL(spec::verify_kernel, dim3(B, 2), dim3(128), 0, static_cast<hipStream_t>(stream), target_probs,
+  hipLaunchKernelGGL(spec::verify_kernel, dim3(B, 2), dim3(spec::kSpecThreads), 0, static_cast<hipStream_t>(stream), target_probs,
                      draft_probs, draft_tokens, random_vals, accepted_count, output_tokens, K, vocab_size);
   return check_launch(fn);
 }

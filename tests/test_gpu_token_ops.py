@@ -233,6 +233,30 @@ def test_speculative_verify_non_monotone_rows(fa):
     _check_spec(fa, tp, dp, tok, rv, K)
 
 
+@pytest.mark.parametrize("V", [511, 512, 513, 8191, 8192, 8193, 16390, 40001])
+def test_speculative_verify_scan_edges(fa, V):
+    """The parallel scans of the serial sums at the edges of their waves (512
+    terms) and tiles (8192): exact (whole tokens) against the serial oracle,
+    with a zero prefix, one term that lifts the sum by many binades, terms on
+    ties, and r on a running sum of the bonus row."""
+    B, K = 6, 1
+    g = torch.Generator().manual_seed(V)
+    tp = torch.softmax(3.0 * torch.randn(B, K + 1, V, generator=g), -1)
+    dp = torch.softmax(3.0 * torch.randn(B, K, V, generator=g), -1)
+    tp[0, :, :V - 3] = 0.0                     # nothing before the last terms
+    tp[1, :, V // 2] = 0.75                    # many binades in one addition
+    tp[2] = torch.randint(0, 9, (K + 1, V), generator=g) * 2.0 ** -18  # ties and exact binade ends
+    dp[2] = torch.randint(0, 5, (K, V), generator=g) * 2.0 ** -19
+    tok = torch.randint(0, V, (B, K), generator=g)
+    rv = torch.rand(B, K, generator=g)
+    rv[5, 0] = 1.0  # rejected; the bonus row's sum may never reach it
+    for b in (3, 4):  # accepted, and r equal to a late running sum of the bonus row
+        tp[b, 0, tok[b, 0]] = 1.0
+        cs = np.cumsum(tp[b, K].numpy().astype(np.float32), dtype=np.float32)
+        rv[b, 0] = float(cs[V - 2 if b == 3 else (2 * V) // 3])
+    _check_spec(fa, tp, dp, tok, rv, K)
+
+
 def test_speculative_verify_validation(fa):
     tp = torch.rand(1, 3, 10, device="cuda")
     dp = torch.rand(1, 2, 10, device="cuda")
