@@ -11,9 +11,11 @@
 //   V   read with ds_read_b64_tr_b16 as the A operand of O^T = V^T P^T
 // Tiles are copied HBM -> LDS by global_load_lds_dwordx4 (no VGPR staging), NS-1
 // tiles ahead of the one being computed, with one barrier per tile; every
-// wave waits (vmcnt) only for its own copies of the current tile.  Shapes the
-// DMA cannot serve (D not 64/128/256 or unaligned rows) stage through registers
-// into the same layout.
+// wave waits (vmcnt) only for its own copies of the current tile.  Rows of
+// whole 16-byte chunks narrower than the tile (D % 8 == 0: 80, 96, 192 ...)
+// are copied the same way with the lanes past D masked off, and the products
+// stop at DC columns.  Shapes the DMA cannot serve (other D, unaligned rows)
+// stage through registers into the same layout.
 //
 // S^T = K Q^T puts one query row per lane (lane l owns query l%32 of each block
 // and 16 keys of each 32-key block): the row max needs one exchange (lanes l,
@@ -40,6 +42,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "capi_internal.h"
 #include "common.h"
@@ -115,7 +118,7 @@ struct PrefillParams {
 // 32w .. 32w + 31; their partial (max, sum, O) merge through LDS at the end.
 // Each wave's serial chain is then a quarter of the keys, which is what bounds
 // short prefills that occupy only a few dozen CUs.
-template <int DP, bool WIDE = false, bool KSPLIT = false>
+template <int DP, bool WIDE = false, bool KSPLIT = false, int DC = DP>
 struct PrefillShape {
   static constexpr int RB = KSPLIT ? 1 : (DP <= 64 ? FA_PRE_RB64 : 1);  // 32-row query blocks per wave
   static constexpr int RW = 32 * RB;                                    // query rows per wave
@@ -125,7 +128,14 @@ struct PrefillShape {
                                    : (DP <= 64 ? (WIDE ? FA_PRE_NSW : 3) : (DP <= 128 ? FA_PRE_NS128 : 2));  // LDS ring stages
   static constexpr int TILE = BK * DP;                                  // halves per K (or V) tile
   static constexpr int WAVES_PER_SIMD =
-      KSPLIT ? 2 : (DP <= 64 ? (WIDE ? 3 : FA_PRE_W64) : (DP <= 128 ? FA_PRE_W128 : 2));  // register budget target
+      KSPLIT ? 2 : (DP <= 64 ? (WIDE ? 3 : FA_PRE_W64) : (DP <= 128 ? (DC <= 96 ? 4 : FA_PRE_W128) : 2));  // register budget target
+};
+
+// How rows reach LDS and the output.
+enum RowMode : int {
+  kRowElems = 0,   // element loads and stores: any D and alignment
+  kRowFull = 1,    // D == DP, 16-byte aligned rows
+  kRowChunks = 2,  // D < DP, D % 8 == 0, 16-byte aligned rows: chunks past D are not copied
 };
 
 // Varlen output rows that no sequence's attention writes are set to zero by
@@ -167,10 +177,12 @@ __device__ __forceinline__ void preload_args(const PrefillParams& p) {
   asm volatile("" ::"s"(p.causal), "s"(p.qtiles), "s"(p.zero_base), "s"(p.group_units), "s"(p.scale_log2));
 }
 
-template <int DP, bool VARLEN, bool VEC, bool WIDE = false, bool KSPLIT = false>
+// DP: padded row width in LDS; DC: columns computed (D <= DC <= DP).
+template <int DP, int DC, bool VARLEN, int ROWS, bool WIDE = false, bool KSPLIT = false>
 __global__ __launch_bounds__(kPreThreads)
-__attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIMD))) void prefill_kernel(PrefillParams p) {
-  using Shape = PrefillShape<DP, WIDE, KSPLIT>;
+__attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER_SIMD))) void prefill_kernel(PrefillParams p) {
+  using Shape = PrefillShape<DP, WIDE, KSPLIT, DC>;
+  constexpr bool VEC = ROWS != kRowElems;
   constexpr int RB = Shape::RB;
   constexpr int RW = Shape::RW;
   constexpr int BQ = Shape::BQ;
@@ -178,8 +190,8 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
   constexpr int NS = Shape::NS;
   constexpr int TILE = Shape::TILE;
   constexpr int NBLK = KSPLIT ? 1 : kBK / 32;  // 32-key blocks per tile computed by one wave
-  constexpr int KK = DP / 16;                 // 16-wide d slices of QK^T
-  constexpr int DB = DP / 32;                 // 32-row d blocks of PV
+  constexpr int KK = DC / 16;                 // 16-wide d slices of QK^T
+  constexpr int DB = (DC + 31) / 32;          // 32-row d blocks of PV
   constexpr int CPR = DP / 8;                 // 16-byte chunks per row
   constexpr int IPW = TILE / 8 / 64 / kPreWaves;  // 16-byte copies per lane per tensor per tile
   constexpr float kRescaleLimit = 256.0f;  // 2^8: largest p before the max is refreshed
@@ -303,8 +315,12 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
       const unsigned slot = sk + (wave * IPW + i) * 1024;
       if constexpr (VEC) {
         const unsigned off = tail ? static_cast<unsigned>((row * stride + cp_col[i]) * sizeof(half_t)) : cp_off[i];
-        copy16_to_lds(kb, off, slot);
-        copy16_to_lds(vb, off, slot + kTileBytes);
+        // every copy instruction covers at least one whole row, so it always
+        // has active lanes and the waves' vmcnt counts hold
+        if (ROWS == kRowFull || cp_col[i] < D) {
+          copy16_to_lds(kb, off, slot);
+          copy16_to_lds(vb, off, slot + kTileBytes);
+        }
       } else {
         const u32x4 kx = load_row8<false>(kb + static_cast<size_t>(row) * stride, cp_col[i], D);
         const u32x4 vx = load_row8<false>(vb + static_cast<size_t>(row) * stride, cp_col[i], D);
@@ -313,6 +329,20 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
       }
     }
   };
+  if constexpr (ROWS == kRowChunks && DC % 32 == 0) {
+    // Chunks past D are never copied.  K's are read up to DC and must not hold
+    // a NaN against Q's zeros; V's only reach output columns past D.
+    if (D < DC) {
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int i = 0; i < IPW; ++i)
+          if (cp_col[i] >= D)
+            *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(
+                static_cast<size_t>(lds_base + t * kStageBytes + (wave * IPW + i) * 1024 + lane * 16)) = zero;
+    }
+  }
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t)
     if (t < ntiles) issue(t);
@@ -325,7 +355,9 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
     const half_t* qr = qp + static_cast<size_t>(min(qrow, rows - 1)) * stride;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      u32x4 x = load_row8<VEC>(qr, kk * 16 + 8 * hi, D);
+      const int qc = kk * 16 + 8 * hi;
+      u32x4 x = u32x4{0u, 0u, 0u, 0u};
+      if (ROWS != kRowChunks || qc < D) x = load_row8<VEC>(qr, qc, D);
       if (qrow >= rows) x = u32x4{0u, 0u, 0u, 0u};
       qf[rb][kk] = __builtin_bit_cast(half8_t, x);
     }
@@ -555,7 +587,7 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
 #pragma unroll
         for (int j = 0; j < 4; ++j) hv[j] = static_cast<half_t>(acc[j] * inv);
         if constexpr (VEC) {
-          *reinterpret_cast<half4_t*>(op + c0 + c) = hv;
+          if (ROWS == kRowFull || c0 + c < D) *reinterpret_cast<half4_t*>(op + c0 + c) = hv;
         } else {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
@@ -589,7 +621,7 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
 #pragma unroll
         for (int j = 0; j < 4; ++j) hv[j] = static_cast<half_t>(oacc[db][rb][4 * rr + j] * inv);
         if constexpr (VEC) {
-          *reinterpret_cast<half4_t*>(op + d0) = hv;
+          if (ROWS == kRowFull || d0 < D) *reinterpret_cast<half4_t*>(op + d0) = hv;
         } else {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
@@ -600,12 +632,21 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT>::WAVES_PER_SIM
   }
 }
 
-template <int DP, bool VARLEN, bool WIDE = false, bool KSPLIT = false>
-static void launch_prefill(bool vec, int blocks, const PrefillParams& p, hipStream_t st) {
-  if (vec)
-    hipLaunchKernelGGL((prefill_kernel<DP, VARLEN, true, WIDE, KSPLIT>), dim3(blocks), dim3(kPreThreads), 0, st, p);
-  else
-    hipLaunchKernelGGL((prefill_kernel<DP, VARLEN, false, WIDE, KSPLIT>), dim3(blocks), dim3(kPreThreads), 0, st, p);
+template <int DP, int DC, bool VARLEN, int ROWS>
+static void launch_shape(bool wide, bool ksplit, int blocks, const PrefillParams& p, hipStream_t st) {
+  if constexpr (DP <= 128) {
+    if (ksplit) {
+      hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS, false, true>), dim3(blocks), dim3(kPreThreads), 0, st, p);
+      return;
+    }
+  }
+  if constexpr (DP <= 64) {
+    if (wide) {
+      hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS, true>), dim3(blocks), dim3(kPreThreads), 0, st, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS>), dim3(blocks), dim3(kPreThreads), 0, st, p);
 }
 constexpr long long kWideMaxBlocks = 1024;  // D <= 64 launches up to this size use 64-key tiles
 // D <= 128 launches of at most this many 128-row workgroups run key-split
@@ -637,15 +678,40 @@ static int dispatch_prefill(const char* fn, int D, bool vec, int rows_max, Prefi
   if (blocks > 0x7fffffffLL) return set_error(FA_ERR_UNSUPPORTED, "%s: problem too large for one launch", fn);
   if (blocks == 0) return FA_OK;
   p.zero_base = static_cast<int>(main_blocks);
-  if (ksplit) {
-    if (D <= 64) launch_prefill<64, VARLEN, false, true>(vec, static_cast<int>(blocks), p, st);
-    else launch_prefill<128, VARLEN, false, true>(vec, static_cast<int>(blocks), p, st);
-  } else if (D <= 64) {
-    if (main_blocks <= kWideMaxBlocks) launch_prefill<64, VARLEN, true>(vec, static_cast<int>(blocks), p, st);
-    else launch_prefill<64, VARLEN>(vec, static_cast<int>(blocks), p, st);
-  }
-  else if (D <= 128) launch_prefill<128, VARLEN>(vec, static_cast<int>(blocks), p, st);
-  else launch_prefill<256, VARLEN>(vec, static_cast<int>(blocks), p, st);
+  // Rows of whole aligned chunks take the DMA, and the products stop at the
+  // narrowest built width that holds D.  Element-staged, D = 80 (8 x 16 heads,
+  // 577 keys, full) took 111 us and computed 128 columns; copied in chunks over
+  // 80 columns it takes 26.3 us (D = 96, causal 4 x 32 x 2048: 604 -> 123 us;
+  // D = 192: 999 -> 245 us; D = 32: 182 -> 65 us).
+  const bool wide = main_blocks <= kWideMaxBlocks;
+  const int n = static_cast<int>(blocks);
+  auto run = [&](auto dp, auto dc, auto mode) {
+    launch_shape<dp(), dc(), VARLEN, mode()>(wide, ksplit, n, p, st);
+  };
+  constexpr std::integral_constant<int, kRowElems> elems;
+  constexpr std::integral_constant<int, kRowFull> full;
+  constexpr std::integral_constant<int, kRowChunks> chunks;
+  constexpr std::integral_constant<int, 32> w32;
+  constexpr std::integral_constant<int, 64> w64;
+  constexpr std::integral_constant<int, 80> w80;
+  constexpr std::integral_constant<int, 96> w96;
+  constexpr std::integral_constant<int, 128> w128;
+  constexpr std::integral_constant<int, 192> w192;
+  constexpr std::integral_constant<int, 256> w256;
+  if (!vec) {
+    if (D <= 64) run(w64, w64, elems);
+    else if (D <= 128) run(w128, w128, elems);
+    else run(w256, w256, elems);
+  } else if (D == 64) run(w64, w64, full);
+  else if (D == 128) run(w128, w128, full);
+  else if (D == 256) run(w256, w256, full);
+  else if (D <= 32) run(w64, w32, chunks);
+  else if (D <= 64) run(w64, w64, chunks);
+  else if (D == 80) run(w128, w80, chunks);
+  else if (D <= 96) run(w128, w96, chunks);
+  else if (D <= 128) run(w128, w128, chunks);
+  else if (D <= 192) run(w256, w192, chunks);
+  else run(w256, w256, chunks);
   return check_launch(fn);
 }
 
@@ -671,8 +737,8 @@ static int prefill_dense(const char* fn, const void* q, const void* k, const voi
   p.B = B; p.H_Q = H_Q; p.H_KV = H_KV; p.N = N; p.D = D; p.G = H_Q / H_KV;
   p.causal = causal ? 1 : 0;
   p.scale_log2 = (1.0f / sqrtf(static_cast<float>(D))) * kLog2e;
-  // Vector path: D fills the padded width exactly and every row starts 16-byte aligned.
-  const bool vec = (D == 64 || D == 128 || D == 256) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
+  // Vector path: rows are whole 16-byte chunks and start 16-byte aligned.
+  const bool vec = D % 8 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
   return dispatch_prefill<false>(fn, D, vec, N, p, static_cast<hipStream_t>(stream));
 }
 
@@ -710,7 +776,7 @@ extern "C" int fa_varlen_prefill_fp16(const void* q, const void* k, const void* 
   p.row_limit = row_limit;
   p.causal = causal ? 1 : 0;
   p.scale_log2 = (1.0f / sqrtf(static_cast<float>(D))) * kLog2e;
-  const bool vec = (D == 64 || D == 128 || D == 256) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
+  const bool vec = D % 8 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
   // Rows past min(row_limit, total) are never computed, so the grid covers that many.
   const int rows_max = row_limit < total ? row_limit : total;
   return dispatch_prefill<true>(fn, D, vec, rows_max, p, static_cast<hipStream_t>(stream));

@@ -1,0 +1,108 @@
+"""Head dims of whole 16-byte chunks that do not fill a padded tile (D % 8 == 0,
+D not 64/128/256): their vector paths against the CPU oracle and against the
+element-wise path, which the same values take from a base that is not 16-byte
+aligned.  The columns past D add exact zeros in both, so results differ by the
+last fp16 rounding at most (one path may fuse the final scaling with the
+conversion, a single rounding in place of two), NaN and infinities alike."""
+import pytest
+import torch
+
+from oracle import attention as A
+from tests.helpers import assert_close, randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def gen(seed):
+    return torch.Generator().manual_seed(seed)
+
+
+def misaligned(t):
+    """The same contiguous values at an address 2 bytes past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)
+    view = buf[1:1 + t.numel()].view(t.shape)
+    view.copy_(t)
+    assert view.data_ptr() % 16 != 0 and view.is_contiguous()
+    return view
+
+
+def equal(a, b):
+    """Same NaN and infinities, and finite values within one fp16 ulp (2^-10 of
+    the value, 2^-24 where it is subnormal)."""
+    a, b = a.float(), b.float()
+    finite = torch.isfinite(a)
+    if not (torch.equal(finite, torch.isfinite(b)) and torch.equal(torch.isnan(a), torch.isnan(b))):
+        return False
+    if not torch.equal(a[torch.isinf(a)], b[torch.isinf(b)]):
+        return False
+    a, b = a[finite], b[finite]
+    return bool(((a - b).abs() <= 2.0 ** -10 * torch.maximum(a.abs(), b.abs()) + 2.0 ** -24).all())
+
+
+DIMS = [8, 24, 32, 40, 72, 80, 88, 96, 104, 120, 160, 192, 200, 248]
+
+
+@pytest.mark.parametrize("d", DIMS)
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("b,hq,hkv,n", [(1, 2, 1, 45),      # key-split workgroups up to D = 128
+                                        (3, 20, 4, 161),    # one round of query tiles
+                                        (2, 16, 16, 577)])
+def test_prefill_chunk_rows(fa, d, causal, b, hq, hkv, n):
+    g = gen(d * 1000 + n)
+    q, k, v = randn(g, b, hq, n, d), randn(g, b, hkv, n, d), randn(g, b, hkv, n, d)
+    qc, kc, vc = (t.to(DEV) for t in (q, k, v))
+    out = fa.forward_prefill_gqa_fp16(qc, kc, vc, causal)
+    assert equal(out, fa.forward_prefill_gqa_fp16(misaligned(qc), kc, vc, causal))
+    if n < 300:
+        assert_close(out, A.prefill(q, k, v, causal), what=f"prefill D={d}")
+
+
+@pytest.mark.parametrize("d", [40, 72, 80, 96, 200])
+def test_prefill_chunk_rows_many_blocks(fa, d):
+    """More query tiles than one residency round (32-key tiles at D <= 64)."""
+    g = gen(d)
+    qc, kc, vc = (randn(g, 8, 32, 600, d).to(DEV) for _ in range(3))
+    assert equal(fa.forward_fp16(qc, kc, vc, True), fa.forward_fp16(misaligned(qc), kc, vc, True))
+
+
+@pytest.mark.parametrize("d", [24, 72, 80, 88, 160])
+def test_prefill_chunk_rows_special_values(fa, d):
+    """Infinities and NaN reach the same outputs whatever LDS held past D."""
+    g = gen(d + 5)
+    q, k, v = (randn(g, 2, 8, 200, d).to(DEV) for _ in range(3))
+    k[0, 1, 50, d - 1] = float("-inf")
+    k[1, 2, 60, 3] = float("inf")
+    v[0, 3, 70, 0] = float("inf")
+    v[1, 4, 80, d - 2] = float("nan")
+    q[0, 5, 90, 1] = float("nan")
+    junk = torch.full((64 << 20,), float("nan"), dtype=torch.float16, device=DEV)  # LDS and memory hold NaN before
+    fa.forward_fp16(junk[:2 * 8 * 200 * 128].view(2, 8, 200, 128), junk[:2 * 8 * 200 * 128].view(2, 8, 200, 128),
+                    junk[:2 * 8 * 200 * 128].view(2, 8, 200, 128), False)
+    for causal in (True, False):
+        out = fa.forward_fp16(q, k, v, causal)
+        assert equal(out, fa.forward_fp16(misaligned(q), k, v, causal))
+        assert not torch.isnan(out[0, 0]).any()
+
+
+@pytest.mark.parametrize("d", [8, 32, 72, 80, 96, 112, 192, 200])
+@pytest.mark.parametrize("causal", [True, False])
+def test_varlen_chunk_rows(fa, d, causal):
+    lens = [5, 0, 200, 37, 1, 129]
+    g = gen(d + 17)
+    cu = torch.tensor([0] + torch.cumsum(torch.tensor(lens), 0).tolist(), dtype=torch.int32)
+    tot = int(cu[-1])
+    q, k, v = (randn(g, tot, 3, d) for _ in range(3))
+    qc, kc, vc, cuc = (t.to(DEV) for t in (q, k, v, cu))
+    out = fa.forward_varlen_prefill_fp16(qc, kc, vc, cuc, 200, causal)
+    assert equal(out, fa.forward_varlen_prefill_fp16(misaligned(qc), kc, vc, cuc, 200, causal))
+    assert_close(out, A.varlen_prefill(q, k, v, cu, 200, causal), what=f"varlen D={d}")
+
+
+@pytest.mark.parametrize("d", [40, 80, 120])
+def test_prefill_lse_chunk_rows(fa, d):
+    g = gen(d + 3)
+    qc, kc, vc = (randn(g, 2, 4, 150, d).to(DEV) for _ in range(3))
+    out, lse = fa.forward_fp16_with_lse(qc, kc, vc, True)
+    out2, lse2 = fa.forward_fp16_with_lse(misaligned(qc), kc, vc, True)
+    assert equal(out, out2) and torch.equal(lse, lse2)
