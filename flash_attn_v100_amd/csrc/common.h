@@ -125,6 +125,13 @@ __device__ __forceinline__ void wait_vmem_stores() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
+// How a kernel reads the rows of its inputs (and writes the output's).
+enum RowMode : int {
+  kRowElems = 0,   // element loads and stores: any D and alignment
+  kRowFull = 1,    // D is the padded width, 16-byte aligned rows
+  kRowChunks = 2,  // D below the padded width, rows of whole aligned 16-byte chunks
+};
+
 // Eight fp16 values starting at column `col` of a row of length `d`, zero past d.
 // VEC: the caller guarantees col + 8 <= d and a 16-byte aligned address, so one
 // unconditional dwordx4 load serves (the kernels use it when d equals their

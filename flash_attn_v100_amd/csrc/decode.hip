@@ -265,12 +265,14 @@ __device__ __forceinline__ int counter_index(int slot) {
   return (slot % kLines) * 32 + slot / kLines;
 }
 
-template <int DP, int GB, int MODE, bool VEC, bool LDSK>
+template <int DP, int GB, int MODE, int ROWS, bool LDSK>
 // Registers are the compiler's choice under the 256-thread bound (94-256
 // VGPRs across the instantiations, none spilling); asking for four waves per
 // SIMD made the INT8 KV cache spill (128 registers) and run 14 % slower.
 __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
     DecodeParams p) {
+  constexpr bool VEC = ROWS != kRowElems;
+  constexpr bool kChunks = ROWS == kRowChunks;
   constexpr int NC = DP / 32;                 // 32-column slices of the QK^T product
   constexpr int LPR = DP / 8;                 // lanes per key row in the row layout
   constexpr int RPW = 64 / LPR;               // rows covered by one row-layout load
@@ -336,6 +338,9 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
   // row layout: lane = (row group rg, 8 columns at col)
   const int rg = lane / LPR;
   const int col = (lane % LPR) * 8;
+  // Rows narrower than DP: lanes past D read the row's last chunk; what they
+  // accumulate are output columns past D, never stored.
+  const int vcol = kChunks ? min(col, D - 8) : col;
 
   const int L = seq_len_of<MODE>(p, b);
   // With absorb_tail (fixed-length calls only) the short remainder past
@@ -450,7 +455,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       u32x4 x = u32x4{0u, 0u, 0u, 0u};
-      if (row_ok) x = load_row8<VEC>(qrow, k_col(c), D);
+      if (row_ok && (!kChunks || k_col(c) < D)) x = load_row8<VEC>(qrow, k_col(c), D);
       qa[c] = __builtin_bit_cast(half8_t, x);
       if constexpr (MODE == kModeInt8) quant8(x, inv_qs, qi8[c][0], qi8[c][1]);
     }
@@ -510,17 +515,31 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
           // page read that page again (masked)
           const half_t* pg = p.k + page_base(t0 + (i * RPC / kPage) * kPage);
           const unsigned off = static_cast<unsigned>((((t0 + r) & (kPage - 1)) * D + lc * 8) * 2);
+          // every copy covers whole rows, so it has active lanes whatever D
+          if (kChunks && lc * 8 >= D) continue;
           if constexpr (kStreamKV) copy16_to_lds_nt(pg, off, dst); else copy16_to_lds(pg, off, dst);
         } else {
           const half_t* kh = p.k + kv_head_base;
           const int t = min(t0 + r, klast);
           const int row = t < p.seg1 ? t : t + p.seg_shift;
           const unsigned off = static_cast<unsigned>((row * D + lc * 8) * 2);
+          if (kChunks && lc * 8 >= D) continue;
           if constexpr (kStreamKV) copy16_to_lds_nt(kh, off, dst); else copy16_to_lds(kh, off, dst);
         }
       }
     }
   };
+  if constexpr (kLdsK && kChunks) {
+    // The copies leave the chunks past D alone; QK^T reads them against Q's
+    // zeros, so they must not hold a NaN.
+#pragma unroll
+    for (int i = 0; i < KCOPIES; ++i) {
+      const int slot = i * 64 + lane;
+      if (((slot % CPR) ^ kswz(slot / CPR)) * 8 >= D)
+        *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(static_cast<size_t>(k_lds + slot * 16)) =
+            u32x4{0u, 0u, 0u, 0u};
+    }
+  }
   // Pipelined walk (continuous batching, and contiguous fp16 decode launches
   // that stage K in LDS): V is staged in a second per-wave LDS buffer by the
   // same kind of copies, lane i of copy u landing its 16 bytes (its own
@@ -543,7 +562,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
       for (int u = 0; u < UV; ++u) {
         const int t = min(t0 + u * RPW + rg, klast);
         const int row = t < p.seg1 ? t : t + p.seg_shift;
-        const unsigned off = static_cast<unsigned>((row * D + col) * 2);
+        const unsigned off = static_cast<unsigned>((row * D + vcol) * 2);
         if constexpr (kStreamKV) copy16_to_lds_nt(vh, off, v_lds + u * 1024);
         else copy16_to_lds(vh, off, v_lds + u * 1024);
       }
@@ -582,7 +601,13 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
         // slices c, c + 1 in one 16-byte load (columns k_col(c) .. +16)
 #pragma unroll
         for (int c = 0; c < NC; c += 2) {
-          const u32x4 x = *reinterpret_cast<const u32x4*>(kh + static_cast<size_t>(t) * D + k_col(c));
+          u32x4 x;
+          if constexpr (kChunks) {  // D % 16 == 0: a pair of slices is inside the row or past it
+            x = *reinterpret_cast<const u32x4*>(kh + static_cast<size_t>(t) * D + min(k_col(c), D - 16));
+            if (k_col(c) >= D) x = u32x4{0u, 0u, 0u, 0u};
+          } else {
+            x = *reinterpret_cast<const u32x4*>(kh + static_cast<size_t>(t) * D + k_col(c));
+          }
           T.k[tt][c] = u32x2{x[0], x[1]};
           T.k[tt][c + 1] = u32x2{x[2], x[3]};
         }
@@ -595,7 +620,17 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
     for (int u = 0; u < UV; ++u) {
       const int t = min(t0 + u * RPW + rg, klast);
       T.vs[u] = p.v_sc[sbase + t];
-      T.v[u] = load_i8x8<VEC>(vh + static_cast<size_t>(t) * D, col, D);
+      T.v[u] = load_i8x8<VEC>(vh + static_cast<size_t>(t) * D, vcol, D);
+    }
+  };
+  // This lane's chunk of slice c of a K row, zero past D.
+  auto k_chunk = [&](const half_t* row, int c) -> u32x4 {
+    const int kc = 32 * c + 8 * q4;
+    if constexpr (kChunks) {
+      const u32x4 x = load_row8<true, kStreamKV>(row, min(kc, D - 8), D);
+      return kc < D ? x : u32x4{0u, 0u, 0u, 0u};
+    } else {
+      return load_row8<VEC, kStreamKV && MODE != kModePaged>(row, kc, D);
     }
   };
   // -- loads: rows past k1 are clamped to k1-1 (always valid memory) and their
@@ -608,13 +643,13 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
         for (int tt = 0; tt < T16; ++tt) {
           const half_t* kr = p.k + page_base(t0 + 16 * tt) + l16 * D;
 #pragma unroll
-          for (int c = 0; c < NC; ++c) T.k[tt][c] = load_row8<VEC>(kr, 32 * c + 8 * q4, D);
+          for (int c = 0; c < NC; ++c) T.k[tt][c] = k_chunk(kr, c);
         }
       }
 #pragma unroll
       for (int u = 0; u < UV; ++u) {
         const int t = t0 + u * RPW;  // RPW divides 16: all rows of this load share a page
-        T.v[u] = load_row8<VEC, kStreamKV>(p.v + page_base(t) + ((t + rg) & (kPage - 1)) * D, col, D);
+        T.v[u] = load_row8<VEC, kStreamKV>(p.v + page_base(t) + ((t + rg) & (kPage - 1)) * D, vcol, D);
       }
     } else {
       const half_t* kh = p.k + kv_head_base;
@@ -625,13 +660,13 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
         for (int tt = 0; tt < T16; ++tt) {
           const int t = row_of(min(t0 + 16 * tt + l16, klast));
 #pragma unroll
-          for (int c = 0; c < NC; ++c) T.k[tt][c] = load_row8<VEC, kStreamKV>(kh + t * D, 32 * c + 8 * q4, D);
+          for (int c = 0; c < NC; ++c) T.k[tt][c] = k_chunk(kh + t * D, c);
         }
       }
 #pragma unroll
       for (int u = 0; u < UV; ++u) {
         const int t = row_of(min(t0 + u * RPW + rg, klast));
-        T.v[u] = load_row8<VEC, kStreamKV>(vh + t * D, col, D);
+        T.v[u] = load_row8<VEC, kStreamKV>(vh + t * D, vcol, D);
       }
     }
   };
@@ -1223,39 +1258,40 @@ static WorkspaceLayout plan_layout(const DecodePlan& pl, int B, int H_Q, int H_K
 // latency-bound small grids (config 2, 256 workgroups: 9.0 -> 9.2 us).
 constexpr int kLdsKMinBlocks = 512;
 
-template <int DP, int GB, int MODE, bool VEC>
+template <int DP, int GB, int MODE, int ROWS>
 static void launch_split(const DecodeParams& p, int blocks, hipStream_t st) {
-  if constexpr ((MODE == kModeDecode || MODE == kModeInt8) && VEC) {
+  if constexpr ((MODE == kModeDecode || MODE == kModeInt8) && ROWS != kRowElems) {
     if (blocks >= kLdsKMinBlocks) {
-      hipLaunchKernelGGL((decode_splitkv_kernel<DP, GB, MODE, VEC, true>), dim3(blocks), dim3(kDecThreads), 0, st, p);
+      hipLaunchKernelGGL((decode_splitkv_kernel<DP, GB, MODE, ROWS, true>), dim3(blocks), dim3(kDecThreads), 0, st, p);
       return;
     }
   }
-  hipLaunchKernelGGL((decode_splitkv_kernel<DP, GB, MODE, VEC, false>), dim3(blocks), dim3(kDecThreads), 0, st, p);
+  hipLaunchKernelGGL((decode_splitkv_kernel<DP, GB, MODE, ROWS, false>), dim3(blocks), dim3(kDecThreads), 0, st, p);
 }
 
-template <int DP, int MODE, bool VEC>
+template <int DP, int MODE, int ROWS>
 static void dispatch_gb(int gb, const DecodeParams& p, int blocks, hipStream_t st) {
   switch (gb) {
-    case 1: launch_split<DP, 1, MODE, VEC>(p, blocks, st); break;
-    case 2: launch_split<DP, 2, MODE, VEC>(p, blocks, st); break;
-    case 4: launch_split<DP, 4, MODE, VEC>(p, blocks, st); break;
-    case 8: launch_split<DP, 8, MODE, VEC>(p, blocks, st); break;
-    default: launch_split<DP, 16, MODE, VEC>(p, blocks, st); break;
+    case 1: launch_split<DP, 1, MODE, ROWS>(p, blocks, st); break;
+    case 2: launch_split<DP, 2, MODE, ROWS>(p, blocks, st); break;
+    case 4: launch_split<DP, 4, MODE, ROWS>(p, blocks, st); break;
+    case 8: launch_split<DP, 8, MODE, ROWS>(p, blocks, st); break;
+    default: launch_split<DP, 16, MODE, ROWS>(p, blocks, st); break;
   }
+}
+
+template <int MODE, int ROWS>
+static void dispatch_dp(const DecodePlan& pl, const DecodeParams& p, int blocks, hipStream_t st) {
+  if (pl.dp == 64) dispatch_gb<64, MODE, ROWS>(pl.gb, p, blocks, st);
+  else if (pl.dp == 128) dispatch_gb<128, MODE, ROWS>(pl.gb, p, blocks, st);
+  else dispatch_gb<256, MODE, ROWS>(pl.gb, p, blocks, st);
 }
 
 template <int MODE>
-static void dispatch(const DecodePlan& pl, bool vec, const DecodeParams& p, int blocks, hipStream_t st) {
-  if (vec) {
-    if (pl.dp == 64) dispatch_gb<64, MODE, true>(pl.gb, p, blocks, st);
-    else if (pl.dp == 128) dispatch_gb<128, MODE, true>(pl.gb, p, blocks, st);
-    else dispatch_gb<256, MODE, true>(pl.gb, p, blocks, st);
-  } else {
-    if (pl.dp == 64) dispatch_gb<64, MODE, false>(pl.gb, p, blocks, st);
-    else if (pl.dp == 128) dispatch_gb<128, MODE, false>(pl.gb, p, blocks, st);
-    else dispatch_gb<256, MODE, false>(pl.gb, p, blocks, st);
-  }
+static void dispatch(const DecodePlan& pl, int rows, const DecodeParams& p, int blocks, hipStream_t st) {
+  if (rows == kRowFull) dispatch_dp<MODE, kRowFull>(pl, p, blocks, st);
+  else if (rows == kRowChunks) dispatch_dp<MODE, kRowChunks>(pl, p, blocks, st);
+  else dispatch_dp<MODE, kRowElems>(pl, p, blocks, st);
 }
 
 static int check_common(const char* fn, int B, int H_Q, int H_KV, int D) {
@@ -1329,15 +1365,21 @@ static int run_decode(const char* fn, DecodeParams p, int max_len, void* ws, siz
     p.ws_lse = reinterpret_cast<float*>(base + wl.lse);
     p.ws_o = reinterpret_cast<float*>(base + wl.o);
   }
-  // Vector path: D fills the padded width exactly and every row starts 16-byte aligned.
-  const bool vec = (p.D == pl.dp) && aligned16(p.q) &&
-                   (MODE == kModeInt8KV ? aligned16(p.k8) && aligned8(p.v8) : aligned16(p.k) && aligned16(p.v));
+  // Vector paths: every row starts 16-byte aligned and is whole 16-byte chunks
+  // (int8 rows: D % 16 == 0), filling the padded width or not.  Read element
+  // by element, 16 x 8 KV heads x 2049 keys took 79 us at D = 80 and 92 us at
+  // D = 96 (1.1 TB/s); in chunks they take 19.8 and 21.0 us (4.2-4.8 TB/s;
+  // D = 128: 24.9 us), paged and INT8 alike.
+  const bool aligned = aligned16(p.q) &&
+                       (MODE == kModeInt8KV ? aligned16(p.k8) && aligned8(p.v8) : aligned16(p.k) && aligned16(p.v));
+  const int chunk = MODE == kModeInt8KV ? 16 : 8;
+  const int rows = !aligned || p.D % chunk != 0 ? kRowElems : (p.D == pl.dp ? kRowFull : kRowChunks);
   const long long units = static_cast<long long>(p.B) * p.H_KV * pl.num_hg;
   hipStream_t st = static_cast<hipStream_t>(stream);
   for (long long u0 = 0; u0 < units; u0 += static_cast<long long>(kCounterSlots)) {
     const long long nu = units - u0 < static_cast<long long>(kCounterSlots) ? units - u0 : kCounterSlots;
     p.unit_base = static_cast<int>(u0);
-    dispatch<MODE>(pl, vec, p, static_cast<int>(nu * pl.splits), st);
+    dispatch<MODE>(pl, rows, p, static_cast<int>(nu * pl.splits), st);
     const int rc = check_launch(fn);
     if (rc != FA_OK) return rc;
   }

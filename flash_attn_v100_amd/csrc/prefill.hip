@@ -131,13 +131,6 @@ struct PrefillShape {
       KSPLIT ? 2 : (DP <= 64 ? (WIDE ? 3 : FA_PRE_W64) : (DP <= 128 ? (DC <= 96 ? 4 : FA_PRE_W128) : 2));  // register budget target
 };
 
-// How rows reach LDS and the output.
-enum RowMode : int {
-  kRowElems = 0,   // element loads and stores: any D and alignment
-  kRowFull = 1,    // D == DP, 16-byte aligned rows
-  kRowChunks = 2,  // D < DP, D % 8 == 0, 16-byte aligned rows: chunks past D are not copied
-};
-
 // Varlen output rows that no sequence's attention writes are set to zero by
 // batch + 1 extra workgroups: workgroup b < batch clears rows
 // [cu[b] + min(len_b, row_limit), cu[b+1]) of sequence b, workgroup batch

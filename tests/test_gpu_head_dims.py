@@ -106,3 +106,71 @@ def test_prefill_lse_chunk_rows(fa, d):
     out, lse = fa.forward_fp16_with_lse(qc, kc, vc, True)
     out2, lse2 = fa.forward_fp16_with_lse(misaligned(qc), kc, vc, True)
     assert equal(out, out2) and torch.equal(lse, lse2)
+
+
+# Query heads per KV head 1..16 pick the kernels' head blocks; B = 40 x 4 KV
+# heads is past the launch size from which contiguous decode stages K in LDS.
+DECODE = [(1, 4, 4, 700), (2, 12, 4, 333), (40, 16, 4, 300), (1, 32, 2, 4100)]
+
+
+@pytest.mark.parametrize("d", [8, 40, 72, 80, 96, 120, 192, 200])
+@pytest.mark.parametrize("b,hq,hkv,n", DECODE)
+def test_decode_chunk_rows(fa, d, b, hq, hkv, n):
+    """Contiguous and sliding-window decode, continuous batching."""
+    g = gen(d * 77 + n)
+    q, k, v = randn(g, b, hq, 1, d), randn(g, b, hkv, n, d), randn(g, b, hkv, n, d)
+    qc, kc, vc = (t.to(DEV) for t in (q, k, v))
+    qm = misaligned(qc)
+    out = fa.forward_decode_gqa_fp16(qc, kc, vc, True, n - 2)
+    assert equal(out, fa.forward_decode_gqa_fp16(qm, kc, vc, True, n - 2))
+    if n < 1000:
+        assert_close(out, A.decode(q, k, v, True, n - 2), what=f"decode D={d}")
+    out = fa.forward_decode_sliding_window_gqa(qc, kc, vc, True, n - 5, n // 2, 9)
+    assert equal(out, fa.forward_decode_sliding_window_gqa(qm, kc, vc, True, n - 5, n // 2, 9))
+    lens = torch.randint(0, n, (b,), generator=g, dtype=torch.int32).to(DEV)
+    out = fa.forward_continuous_batching_fp16(qc, kc, vc, lens, True)
+    assert equal(out, fa.forward_continuous_batching_fp16(qm, kc, vc, lens, True))
+
+
+@pytest.mark.parametrize("d", [8, 40, 72, 80, 96, 120, 192, 200])
+@pytest.mark.parametrize("b,hq,hkv,n", DECODE)
+def test_paged_and_int8_decode_chunk_rows(fa, d, b, hq, hkv, n):
+    g = gen(d * 79 + n)
+    blocks = (n + 15) // 16
+    pages = b * blocks + 3
+    q = randn(g, b, hq, 1, d).to(DEV)
+    qm = misaligned(q)
+    kp, vp = randn(g, pages, hkv, 16, d).to(DEV), randn(g, pages, hkv, 16, d).to(DEV)
+    table = torch.randperm(pages, generator=g)[:b * blocks].to(torch.int32).view(b, blocks).to(DEV)
+    lens = torch.randint(1, n + 1, (b,), generator=g, dtype=torch.int32).to(DEV)
+    out = fa.forward_paged_decode_gqa_fp16(q, kp, vp, table, lens, blocks)
+    assert equal(out, fa.forward_paged_decode_gqa_fp16(qm, kp, vp, table, lens, blocks))
+
+    k, v = randn(g, b, hkv, n, d).to(DEV), randn(g, b, hkv, n, d).to(DEV)
+    qs = q.float().abs().amax((2, 3)) / 127.0
+    ks = (k.float().abs().amax((2, 3)) / 127.0)[..., None].expand(b, hkv, n).contiguous()
+    out = fa.forward_decode_int8_gqa(q, k, v, qs, ks, n - 1)
+    assert equal(out, fa.forward_decode_int8_gqa(qm, k, v, qs, ks, n - 1))
+
+    k8 = torch.randint(-127, 128, (b, hkv, n, d), generator=g, dtype=torch.int8).to(DEV)
+    v8 = torch.randint(-127, 128, (b, hkv, n, d), generator=g, dtype=torch.int8).to(DEV)
+    s1 = (torch.rand(b, hkv, n, generator=g) * 0.03).half().to(DEV)
+    s2 = (torch.rand(b, hkv, n, generator=g) * 0.03).half().to(DEV)
+    out = fa.forward_decode_int8_kv_cache_gqa(q, k8, v8, s1, s2, n - 1)
+    assert equal(out, fa.forward_decode_int8_kv_cache_gqa(qm, k8, v8, s1, s2, n - 1))
+
+
+@pytest.mark.parametrize("d", [72, 80, 200])
+@pytest.mark.parametrize("b,hq,hkv,n", [(1, 4, 2, 200), (40, 16, 4, 300)])
+def test_decode_chunk_rows_special_values(fa, d, b, hq, hkv, n):
+    """Infinities and NaN of a cache reach the same outputs on both paths."""
+    g = gen(d)
+    q, k, v = randn(g, b, hq, 1, d).to(DEV), randn(g, b, hkv, n, d).to(DEV), randn(g, b, hkv, n, d).to(DEV)
+    k[0, 0, 40, d - 1] = float("-inf")
+    v[0, 1, 70, 0] = float("nan")
+    v[0, 1, 71, d - 1] = float("inf")
+    lens = torch.full((b,), n - 1, dtype=torch.int32, device=DEV)
+    qm = misaligned(q)
+    assert equal(fa.forward_decode_gqa_fp16(q, k, v, True, n - 1), fa.forward_decode_gqa_fp16(qm, k, v, True, n - 1))
+    assert equal(fa.forward_continuous_batching_fp16(q, k, v, lens, True),
+                 fa.forward_continuous_batching_fp16(qm, k, v, lens, True))
