@@ -90,7 +90,6 @@ extern "C" int fa_prefill_fp32(const void* q, const void* k, const void* v, void
   TrainParams p = {};
   p.q = q; p.k = k; p.v = v; p.out = o; p.lse = lse;
   p.BH = B * H; p.N = N; p.D = D; p.causal = causal ? 1 : 0;
-  p.nblk = ceil_div(N, kBlockRows);
   p.scale = 1.0f / sqrtf(static_cast<float>(D));
   p.scale_log2 = p.scale * kLog2e;
   const bool vec = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o);
@@ -121,7 +120,6 @@ static int backward_common(const char* fn, bool fp32, const void* dout, const vo
   p.lse = const_cast<float*>(lse);
   p.delta = static_cast<float*>(workspace);
   p.BH = B * H; p.N = N; p.D = D; p.causal = causal ? 1 : 0;
-  p.nblk = ceil_div(N, kBlockRows);
   p.scale = 1.0f / sqrtf(static_cast<float>(D));
   p.scale_log2 = p.scale * kLog2e;
   const bool vec = aligned16(dout) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) &&

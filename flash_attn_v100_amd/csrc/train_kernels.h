@@ -36,9 +36,9 @@
 // ahead, one barrier per tile.  fp32 tiles and odd D stage through registers
 // into a two-stage ring (fp32 rows padded by 32 bytes).
 //
-// The backward runs on one stream: dQ first (each wave also computes
-// delta_i = sum_d dO[i,d] O[i,d] of its rows and publishes it in the
-// workspace), then dK/dV, which reads delta.  The key-major kernel does both
+// The backward is dQ (each wave also computes delta_i = sum_d dO[i,d] O[i,d] of
+// its rows and publishes it in the workspace), then dK/dV, which reads delta;
+// large calls fork the passes onto side streams (backward_plan).  The key-major kernel does both
 // dK and dV in one pass when its registers allow (fp32, D <= 64 in fp16);
 // otherwise (fp16, D > 64) one pass does dV (S and P only) and another dK
 // (S, dP, dS), so each fits 256 VGPRs and two waves share a SIMD.  No atomics:
@@ -92,7 +92,7 @@ template <typename T, int DP>
 struct Layout;
 template <int DP>
 struct Layout<half_t, DP> {  // unpadded, 16-byte chunks XOR-swizzled per row
-  static constexpr int TILE = kRows * DP;
+  static constexpr int LD = DP;
   __device__ static __forceinline__ int off(int r, int c) {
     return r * DP + ((((c >> 3) ^ chunk_swizzle<DP>(r)) << 3) | (c & 7));
   }
@@ -100,7 +100,6 @@ struct Layout<half_t, DP> {  // unpadded, 16-byte chunks XOR-swizzled per row
 template <int DP>
 struct Layout<float, DP> {  // rows padded by 32 bytes (8 banks apart mod 64)
   static constexpr int LD = DP + 8;
-  static constexpr int TILE = kRows * LD;
   __device__ static __forceinline__ int off(int r, int c) { return r * LD + c; }
 };
 
@@ -161,27 +160,30 @@ struct Reader<float, DP> {
 };
 
 // Eight elements of global row `row` (length d) from column `col`, zero past d;
-// VEC: d == padded width and 16-byte aligned rows, so one vector load serves.
-template <typename T, bool VEC>
-__device__ __forceinline__ typename Elem<T>::frag load_frag(const T* row, int col, int d) {
-  typedef typename Elem<T>::frag F;
-  if constexpr (VEC) {
-    (void)d;
-    return *reinterpret_cast<const F*>(row + col);
-  } else {
-    F f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = (col + j < d) ? row[col + j] : static_cast<T>(0.0f);
-    return f;
-  }
-}
-
+// the vector row modes have 16-byte aligned rows of whole 8-element groups, so
+// one vector load serves (kRowFull: d is the padded width).
 template <typename T>
 __device__ __forceinline__ typename Elem<T>::frag zero_frag() {
   typename Elem<T>::frag f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) f[j] = static_cast<T>(0.0f);
   return f;
+}
+
+template <typename T, int ROWS>
+__device__ __forceinline__ typename Elem<T>::frag load_frag(const T* row, int col, int d) {
+  typedef typename Elem<T>::frag F;
+  if constexpr (ROWS == kRowFull) {
+    (void)d;
+    return *reinterpret_cast<const F*>(row + col);
+  } else if constexpr (ROWS == kRowChunks) {
+    return col < d ? *reinterpret_cast<const F*>(row + col) : zero_frag<T>();
+  } else {
+    F f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = (col + j < d) ? row[col + j] : static_cast<T>(0.0f);
+    return f;
+  }
 }
 
 // Operand slice `sl` (accumulator registers 8 sl .. 8 sl + 7) converted to T.
@@ -193,28 +195,32 @@ __device__ __forceinline__ typename Elem<T>::frag acc_frag(const float16_t& a, i
   return f;
 }
 
-// Streams 32-row tiles of two [N, D] row-major tensors (and, with VECS, two
+// Streams SR-row tiles of two [N, D] row-major tensors (and, with VECS, two
 // per-row float vectors) through an LDS ring.  A stage holds
-//   [tensor A tile | tensor B tile | VECS: 64 floats of vector 0 | 64 of vector 1]
-// (only the first 32 floats of each vector slot are used).
-//  DMA (fp16, D = DP, 16-byte aligned rows): stages filled by global_load_lds,
-//    one tile ahead; rows past `rows` re-read the last row (callers mask them).
+//   [tensor A tile | tensor B tile | VECS: VSLOT floats of vector 0 | VSLOT of vector 1]
+// (only the first SR floats of each vector slot are used).
+//  DMA (fp16, rows of whole 16-byte aligned chunks): stages filled by
+//    global_load_lds, one tile ahead; rows past `rows` re-read the last row
+//    (callers mask them); chunks past d are zeroed once and never copied.
 //  otherwise: stages filled through registers; rows past `rows` are 0
 //    and vector 0 / vector 1 read +inf / 0 there.
 // Vector 0 is stored pre-multiplied by log2(e) on the register path only; DMA
 // consumers scale at the read (vec_scale()).
-template <typename T, int DP, bool DMA, bool VECS>
+template <typename T, int DP, bool DMA, bool VECS, int SR_, int ROWS>
 struct TileRing {
   typedef typename Elem<T>::frag F;
   typedef Layout<T, DP> L;
+  static constexpr int SR = SR_;
   static constexpr int NS = 2;  // three DMA stages measured 4.7 % slower (config 7 backward 367 vs 350 us)
-  static constexpr int VEC_FLOATS = VECS ? 128 : 0;
-  static constexpr int STAGE_BYTES = 2 * L::TILE * static_cast<int>(sizeof(T)) + VEC_FLOATS * 4;
+  static constexpr int VSLOT = SR < 64 ? 64 : SR;
+  static constexpr int VEC_FLOATS = VECS ? 2 * VSLOT : 0;
+  static constexpr int TILE_BYTES = SR * L::LD * static_cast<int>(sizeof(T));
+  static constexpr int STAGE_BYTES = 2 * TILE_BYTES + VEC_FLOATS * 4;
   static constexpr int BYTES = NS * STAGE_BYTES;
   static constexpr int CPR = DP / 8;            // 8-element groups per row
-  static constexpr int CHUNKS = kRows * CPR;    // groups per tile
+  static constexpr int CHUNKS = SR * CPR;       // groups per tile
   static constexpr int PER_THREAD = (CHUNKS + kThreads - 1) / kThreads;
-  // DMA instructions this wave issues per tile (waves 0 and 1 also copy a vector)
+  // DMA instructions this wave issues per tile (the first 2 * VSLOT / 64 waves also copy a vector part)
   static constexpr int DMA_PER_TILE = 2 * PER_THREAD;
 
   unsigned lds_base;  // byte address of stage 0
@@ -222,8 +228,8 @@ struct TileRing {
   // register path staging
   F a[DMA ? 1 : PER_THREAD], b[DMA ? 1 : PER_THREAD];
   float v0 = 0.0f, v1 = 0.0f;
-  // DMA path: per copy, the tile row and byte offset of this lane's chunk
-  int cp_row[PER_THREAD];
+  // DMA path: per copy, the tile row, column and byte offset of this lane's chunk
+  int cp_row[PER_THREAD], cp_col[PER_THREAD];
   unsigned cp_off[PER_THREAD];
 
   __device__ TileRing(void* smem, int tid_, int d)
@@ -237,30 +243,43 @@ struct TileRing {
         // (g % CPR) ^ swizzle(row) of row g / CPR
         const int g = i * kThreads + tid;
         cp_row[i] = g / CPR;
-        const int lc = (g % CPR) ^ chunk_swizzle<DP>(g / CPR);
-        cp_off[i] = static_cast<unsigned>((cp_row[i] * d + lc * 8) * 2);
+        cp_col[i] = ((g % CPR) ^ chunk_swizzle<DP>(g / CPR)) * 8;
+        cp_off[i] = static_cast<unsigned>((cp_row[i] * d + cp_col[i]) * 2);
+      }
+      if constexpr (ROWS == kRowChunks) {
+        // chunks past d are products' zeros: they must not hold a NaN
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i)
+          if (cp_col[i] >= d)
+#pragma unroll
+            for (int s = 0; s < 2 * NS; ++s)
+              *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(static_cast<size_t>(
+                  lds_base + (s >> 1) * STAGE_BYTES + (s & 1) * TILE_BYTES + (i * kThreads + tid) * 16)) =
+                  u32x4{0u, 0u, 0u, 0u};
       }
     }
   }
   __device__ __forceinline__ unsigned addr_a(int stage) const { return lds_base + stage * STAGE_BYTES; }
-  __device__ __forceinline__ unsigned addr_b(int stage) const { return addr_a(stage) + L::TILE * sizeof(T); }
+  __device__ __forceinline__ unsigned addr_b(int stage) const { return addr_a(stage) + TILE_BYTES; }
   __device__ __forceinline__ lds_ptr<T> tile_a(int stage) const {
-    return reinterpret_cast<lds_ptr<T>>(static_cast<size_t>(lds_base + stage * STAGE_BYTES));
+    return reinterpret_cast<lds_ptr<T>>(static_cast<size_t>(addr_a(stage)));
   }
-  __device__ __forceinline__ lds_ptr<T> tile_b(int stage) const { return tile_a(stage) + L::TILE; }
+  __device__ __forceinline__ lds_ptr<T> tile_b(int stage) const {
+    return reinterpret_cast<lds_ptr<T>>(static_cast<size_t>(addr_b(stage)));
+  }
   __device__ __forceinline__ const __attribute__((address_space(3))) float* vec(int stage, int which) const {
     return reinterpret_cast<const __attribute__((address_space(3))) float*>(
-        static_cast<size_t>(lds_base + stage * STAGE_BYTES + 2 * L::TILE * sizeof(T) + which * 256));
+        static_cast<size_t>(addr_a(stage) + 2 * TILE_BYTES + which * VSLOT * 4));
   }
 
-  // DMA path: copy rows [r0, r0 + 32) of pa/pb (row stride d == DP) and, with
-  // VECS, va/vb[r0 .. r0 + 32) into `stage`.
+  // DMA path: copy rows [r0, r0 + SR) of pa/pb (row stride d) and, with
+  // VECS, va/vb[r0 .. r0 + SR) into `stage`.
   __device__ __forceinline__ void dma(const T* pa, const T* pb, const float* va, const float* vb, int r0, int rows,
                                       int d, int stage) const {
     const T* ba = pa + static_cast<size_t>(r0) * d;
     const T* bb = pb + static_cast<size_t>(r0) * d;
     const unsigned sbase = lds_base + stage * STAGE_BYTES;
-    const bool tail = r0 + kRows > rows;
+    const bool tail = r0 + SR > rows;
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i) {
       unsigned off = cp_off[i];
@@ -269,21 +288,25 @@ struct TileRing {
         off = static_cast<unsigned>(static_cast<int>(off) + (row - cp_row[i]) * d * 2);
       }
       const unsigned slot = sbase + (i * kThreads + wave * 64) * 16;
-      copy16_to_lds(reinterpret_cast<const half_t*>(ba), off, slot);
-      copy16_to_lds(reinterpret_cast<const half_t*>(bb), off, slot + L::TILE * sizeof(T));
+      // (a copy covers whole rows: it has active lanes whatever d, so vmcnt counts hold)
+      if (ROWS == kRowFull || cp_col[i] < d) {
+        copy16_to_lds(reinterpret_cast<const half_t*>(ba), off, slot);
+        copy16_to_lds(reinterpret_cast<const half_t*>(bb), off, slot + TILE_BYTES);
+      }
     }
     if constexpr (VECS) {
-      if (wave < 2) {
-        const float* base = (wave == 0 ? va : vb) + r0;
-        const unsigned off = static_cast<unsigned>(min(lane & 31, rows - 1 - r0)) * 4;
-        copy4_to_lds(base, off, sbase + 2 * L::TILE * sizeof(T) + wave * 256);
+      if (wave < 2 * VSLOT / 64) {  // wave w: 64 rows from 64 (w / 2) of vector w % 2
+        const float* base = ((wave & 1) ? vb : va) + r0;
+        const int row = SR < 64 ? (lane & (SR - 1)) : lane + 64 * (wave >> 1);
+        const unsigned off = static_cast<unsigned>(min(row, rows - 1 - r0)) * 4;
+        copy4_to_lds(base, off, sbase + 2 * TILE_BYTES + (wave & 1) * (VSLOT * 4) + (wave >> 1) * 256);
       }
     }
   }
   // Waits until this wave's copies of every tile but the newest `pending` ones
   // have landed (DMA path).
   __device__ __forceinline__ void wait_dma(bool one_pending) const {
-    const bool extra = VECS && wave < 2;
+    const bool extra = VECS && wave < 2 * VSLOT / 64;
     if (one_pending) {
       if (extra) wait_vm_lgkm0<DMA_PER_TILE + 1>();
       else wait_vm_lgkm0<DMA_PER_TILE>();
@@ -292,8 +315,7 @@ struct TileRing {
     }
   }
 
-  // Register path: load rows [r0, r0 + 32) (zero past `rows`) into registers ...
-  template <bool VEC>
+  // Register path: load rows [r0, r0 + SR) (zero past `rows`) into registers ...
   __device__ __forceinline__ void load(const T* pa, const T* pb, const float* va, const float* vb, int r0, int rows,
                                        int d) {
 #pragma unroll
@@ -302,15 +324,15 @@ struct TileRing {
       const int row = c / CPR;
       const int col = (c % CPR) * 8;
       if ((CHUNKS % kThreads == 0 || c < CHUNKS) && r0 + row < rows) {
-        a[i] = load_frag<T, VEC>(pa + static_cast<size_t>(r0 + row) * d, col, d);
-        b[i] = load_frag<T, VEC>(pb + static_cast<size_t>(r0 + row) * d, col, d);
+        a[i] = load_frag<T, ROWS>(pa + static_cast<size_t>(r0 + row) * d, col, d);
+        b[i] = load_frag<T, ROWS>(pb + static_cast<size_t>(r0 + row) * d, col, d);
       } else {
         a[i] = zero_frag<T>();
         b[i] = zero_frag<T>();
       }
     }
     if constexpr (VECS) {
-      if (tid < kRows) {
+      if (tid < SR) {
         const int r = r0 + tid;
         v0 = r < rows ? va[r] * kLog2e : INFINITY;  // padding rows: P = 0
         v1 = r < rows ? vb[r] : 0.0f;
@@ -332,10 +354,10 @@ struct TileRing {
       }
     }
     if constexpr (VECS) {
-      if (tid < kRows) {
+      if (tid < SR) {
         auto* v = const_cast<__attribute__((address_space(3))) float*>(vec(stage, 0));
         v[tid] = v0;
-        v[64 + tid] = v1;
+        v[VSLOT + tid] = v1;
       }
     }
   }
@@ -365,7 +387,8 @@ struct TrainParams {
   float* delta;      // backward workspace [B*H*N]
   int delta_ready;   // dQ kernel: delta is already in the workspace (read it, do not recompute)
   int BH, N, D, causal;
-  int nblk;          // 128-row blocks per (batch, head)
+  int nblk;          // row blocks (one workgroup each) per (batch, head)
+  int order;         // BlockOrder
   float scale;       // 1/sqrt(D)
   float scale_log2;  // scale * log2(e)
 };
@@ -379,10 +402,19 @@ struct TrainParams {
 constexpr int kBwdGroupUnits = FA_BWD_GROUP;
 __host__ __device__ inline int bwd_group_units(const TrainParams& p) { return p.causal ? kBwdGroupUnits : 1; }
 
-// Workgroup -> ((batch, head) unit bh, 128-row block blk).  With at least 8
+// Order of a group's blocks on its XCD.  Heavy first suits grids that the
+// dispatcher refills as workgroups end.  Where the whole grid is resident at
+// once, workgroups i and i + 32 of an XCD share a CU (32 CUs an XCD), and heavy
+// first puts the heaviest of each round on the same CUs: the snake order walks
+// every other round of 32 backwards, so each CU gets about the same work (fp32
+// forward with LSE, causal [2,16,1000,64]: 82 us heavy first, 49 us as a snake).
+enum BlockOrder : int { kHeavyFirst = 0, kLightFirst = 1, kSnake = 2 };
+constexpr int kXcdCus = 32;
+
+// Workgroup -> ((batch, head) unit bh, row block blk).  With at least 8
 // units, every block of a unit runs on one XCD (the dispatcher deals workgroup
 // j to XCD j % 8), so the unit's streamed tiles are shared through that XCD's
-// L2, and an XCD walks its units group by group, heaviest block first
+// L2, and an XCD walks its units group by group, heaviest block first (or p.order)
 // (heavy_last: the last block carries the most work).  Returns false for the
 // padding workgroups of the last round.
 __device__ __forceinline__ bool map_block(const TrainParams& p, bool heavy_last, int& bh, int& blk) {
@@ -392,7 +424,14 @@ __device__ __forceinline__ bool map_block(const TrainParams& p, bool heavy_last,
   if (p.BH >= 8) {
     const int i = j / 8;
     const int gu = bwd_group_units(p);
-    const int group = i / (gu * nb), ii = i % (gu * nb);
+    const int group = i / (gu * nb);
+    const int n = gu * nb;
+    int ii = i % n;
+    if (p.order == kLightFirst) ii = n - 1 - ii;
+    if (p.order == kSnake && ((ii / kXcdCus) & 1)) {
+      const int first = ii / kXcdCus * kXcdCus;
+      ii = first + min(n, first + kXcdCus) - 1 - ii;
+    }
     bh = j % 8 + 8 * (group * gu + ii % gu);
     b = ii / gu;
     if (bh >= p.BH) return false;
@@ -418,7 +457,7 @@ inline int train_grid(const TrainParams& p) {
 // tile's index from r_first): workgroups that share a stream but start at
 // different tiles and end together then read each tile at about the same
 // time, so the copies after the first hit L2.
-template <typename Ring, bool DMA, bool VEC, bool REV = false, typename T, typename Compute>
+template <typename Ring, bool DMA, bool REV = false, typename T, typename Compute>
 __device__ __forceinline__ void run_ring(Ring& ring, const T* pa, const T* pb, const float* va, const float* vb,
                                          int r_first, int ntiles, int c_begin, int c_end, int rows, int d,
                                          Compute&& compute) {
@@ -430,7 +469,7 @@ __device__ __forceinline__ void run_ring(Ring& ring, const T* pa, const T* pb, c
     c_begin = b;
   }
   auto tile_of = [&](int t) { return REV ? ntiles - 1 - t : t; };  // stream position -> tile
-  auto row_of = [&](int t) { return r_first + tile_of(t) * kRows; };
+  auto row_of = [&](int t) { return r_first + tile_of(t) * Ring::SR; };
   if constexpr (DMA) {
     constexpr int NS = Ring::NS;
 #pragma unroll
@@ -449,11 +488,11 @@ __device__ __forceinline__ void run_ring(Ring& ring, const T* pa, const T* pb, c
     for (int t = c_end; t < ntiles; ++t) step(t);
   } else {
     if (ntiles > 0) {
-      ring.template load<VEC>(pa, pb, va, vb, row_of(0), rows, d);
+      ring.load(pa, pb, va, vb, row_of(0), rows, d);
       ring.store(0);
     }
     auto pre = [&](int t) {
-      if (t + 1 < ntiles) ring.template load<VEC>(pa, pb, va, vb, row_of(t + 1), rows, d);
+      if (t + 1 < ntiles) ring.load(pa, pb, va, vb, row_of(t + 1), rows, d);
       __syncthreads();
     };
     auto post = [&](int t) {
@@ -475,27 +514,44 @@ __device__ __forceinline__ void run_ring(Ring& ring, const T* pa, const T* pb, c
   }
 }
 
+// Split walks: SPLIT waves of a workgroup share one 32-row block and take the
+// 32-row sub-tiles of every streamed SPLIT * 32-row tile in turn (wave w:
+// block w % (4 / SPLIT), sub-tile w / (4 / SPLIT)); their partial accumulators
+// meet in LDS at the end.  A wave's serial walk is then 1 / SPLIT as long and
+// there are SPLIT times as many workgroups, which is what bounds calls whose
+// 128-row blocks are few.  All of a row block's waves hold the same element in
+// the same lane and register, so partials pass lane to lane: slot
+// [wave][register][lane], conflict-free.
+template <int REGS>
+__device__ __forceinline__ lds_ptr<float> part_slot(char* smem, int wave, int lane) {
+  return reinterpret_cast<lds_ptr<float>>(static_cast<size_t>(static_cast<unsigned>(
+             reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)))) + wave * REGS * 64 + lane;
+}
+
 // ---------------------------------------------------------------------------
 // Query-major kernel: MODE 0 = fp32 forward (O, optional LSE), MODE 1 = dQ + delta.
-template <typename T, int DP, bool VEC, int MODE>
-__global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
+// DC: columns computed (D <= DC <= DP).
+template <typename T, int DP, int DC, int ROWS, int MODE, int SPLIT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && DP <= 64 ? 2 : 1))) void query_major_kernel(TrainParams p) {
   typedef typename Elem<T>::frag F;
-  constexpr int KK = DP / 16;  // 16-deep reduction steps over d
-  constexpr int DB = DP / 32;  // 32-row blocks of d in the transposed products
-  constexpr bool DMA = VEC && sizeof(T) == 2;
-  typedef TileRing<T, DP, DMA, false> Ring;
+  constexpr int KK = DC / 16;         // 16-deep reduction steps over d
+  constexpr int DB = (DC + 31) / 32;  // 32-row blocks of d in the transposed products
+  constexpr bool DMA = ROWS != kRowElems && sizeof(T) == 2;
+  constexpr int RW = kWaves / SPLIT;  // 32-row blocks per workgroup
+  typedef TileRing<T, DP, DMA, false, kRows * SPLIT, ROWS> Ring;
   __shared__ __attribute__((aligned(1024))) char smem[Ring::BYTES];
 
   const int N = p.N, D = p.D;
   int bh, blk;
   if (!map_block(p, p.causal != 0, bh, blk)) return;
-  const int q0 = blk * kBlockRows;
+  const int q0 = blk * (RW * kRows);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int hi = lane >> 5;
-  const int wq0 = q0 + wave * kRows;
+  const int sub = wave / RW;  // sub-tile of each streamed tile this wave computes
+  const int wq0 = q0 + (wave % RW) * kRows;
   const int qrow = wq0 + l32;
   const bool qvalid = qrow < N;
   const size_t base = static_cast<size_t>(bh) * N * D;
@@ -509,7 +565,7 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
   {
     const T* qr = qp + static_cast<size_t>(min(qrow, N - 1)) * D;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) qf[kk] = qvalid ? load_frag<T, VEC>(qr, 16 * kk + 8 * hi, D) : zero_frag<T>();
+    for (int kk = 0; kk < KK; ++kk) qf[kk] = qvalid ? load_frag<T, ROWS>(qr, 16 * kk + 8 * hi, D) : zero_frag<T>();
   }
   if constexpr (MODE == 1) {
     const T* dr = static_cast<const T*>(p.dout) + base + static_cast<size_t>(min(qrow, N - 1)) * D;
@@ -517,9 +573,9 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
     float part = 0.0f;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      df[kk] = qvalid ? load_frag<T, VEC>(dr, 16 * kk + 8 * hi, D) : zero_frag<T>();
+      df[kk] = qvalid ? load_frag<T, ROWS>(dr, 16 * kk + 8 * hi, D) : zero_frag<T>();
       if (!p.delta_ready) {
-        const F of = qvalid ? load_frag<T, VEC>(orow, 16 * kk + 8 * hi, D) : zero_frag<T>();
+        const F of = qvalid ? load_frag<T, ROWS>(orow, 16 * kk + 8 * hi, D) : zero_frag<T>();
 #pragma unroll
         for (int j = 0; j < 8; ++j) part = fmaf(static_cast<float>(df[kk][j]), static_cast<float>(of[j]), part);
       }
@@ -527,7 +583,7 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
     delta = part + __shfl_xor(part, 32, 64);
     if (qvalid) {
       if (p.delta_ready) delta = p.delta[static_cast<size_t>(bh) * N + qrow];  // the same value, from delta_kernel
-      else if (hi == 0) p.delta[static_cast<size_t>(bh) * N + qrow] = delta;
+      else if (hi == 0 && sub == 0) p.delta[static_cast<size_t>(bh) * N + qrow] = delta;
       lse2 = p.lse[static_cast<size_t>(bh) * N + qrow] * kLog2e;
     } else {
       lse2 = INFINITY;  // padding rows: P = 0
@@ -542,19 +598,21 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
   float m_run = kNegBig, l_run = 0.0f;  // forward only (log2 domain)
   const float c = p.scale_log2;
 
-  const int kend = p.causal ? min(N, q0 + kBlockRows) : N;  // keys this workgroup needs
+  const int kend = p.causal ? min(N, q0 + RW * kRows) : N;  // keys this workgroup needs
   // keys this wave needs (none when all its rows lie past N)
   const int kend_w = wq0 >= N ? 0 : (p.causal ? min(N, wq0 + kRows) : N);
-  const int ntiles = (kend + kRows - 1) / kRows;
+  constexpr int SR = Ring::SR;
+  const int ntiles = (kend + SR - 1) / SR;
 
   Ring ring(smem, tid, D);
   const Reader<T, DP> rd(lane);
-  // this wave computes key tiles [0, ceil(kend_w / 32)): later ones are past its diagonal
-  run_ring<Ring, DMA, VEC>(ring, kp, vp, nullptr, nullptr, 0, ntiles, 0, (kend_w + kRows - 1) / kRows, N, D,
-                           [&](int stage, int t) {
-    const int kt = t * kRows;
-    const unsigned ks = ring.addr_a(stage);
-    const unsigned vs = ring.addr_b(stage);
+  constexpr unsigned kSubBytes = kRows * Layout<T, DP>::LD * sizeof(T);
+  // this wave computes its sub-tiles that start before kend_w: later ones are past its diagonal
+  run_ring<Ring, DMA>(ring, kp, vp, nullptr, nullptr, 0, ntiles, 0, (kend_w - sub * kRows + SR - 1) / SR, N, D,
+                      [&](int stage, int t) {
+    const int kt = t * SR + sub * kRows;
+    const unsigned ks = ring.addr_a(stage) + sub * kSubBytes;
+    const unsigned vs = ring.addr_b(stage) + sub * kSubBytes;
     // S^T = K Q^T: lane <-> query, register r <-> key kt + 8 (r/4) + 4 hi + r%4
     float16_t s;
 #pragma unroll
@@ -571,24 +629,37 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
     }
     float16_t pm;  // P^T (forward) or dS^T (dQ)
     if constexpr (MODE == 0) {
-      float mx = s[0];
-#pragma unroll
-      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c;
-      const float mn = fmaxf(m_run, mx);
-      const float alpha = fast_exp2(m_run - mn);
-      m_run = mn;
+      // p = exp2(s c - m) against the running max m, which is only refreshed
+      // (and O, l rescaled) when a lane's partial sum passes 2^8, i.e. some
+      // score outgrew m by more than the slack (always so from m = -1e30).
+      constexpr float kRescaleLimit = 256.0f;
       float ls = 0.0f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        pm[r] = fast_exp2(fmaf(s[r], c, -mn));
+        pm[r] = fast_exp2(fmaf(s[r], c, -m_run));
         ls += pm[r];
       }
-      l_run = fmaf(l_run, alpha, ls);
+      if (__builtin_amdgcn_ballot_w64(!(ls <= kRescaleLimit)) != 0) {
+        float mx = s[0];
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c;
+        const float mn = fmaxf(m_run, mx);
+        const float alpha = fast_exp2(m_run - mn);
+        m_run = mn;
+        l_run *= alpha;
+        ls = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        for (int r = 0; r < 16; ++r) {
+          pm[r] = fast_exp2(fmaf(s[r], c, -mn));
+          ls += pm[r];
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+      }
+      l_run += ls;
     } else {
       // dP^T = V dO^T
       float16_t dp;
@@ -609,6 +680,45 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
     }
   });
 
+  // ---- join the row block's waves: wave `sub` 0 takes the others' partials ----
+  if constexpr (SPLIT > 1) {
+    constexpr int REGS = 16 * DB + (MODE == 0 ? 2 : 0);
+    static_assert((SPLIT - 1) * RW * REGS * 256 <= Ring::BYTES, "partials fit the ring");
+    __syncthreads();  // every wave is done reading the ring
+    if (sub > 0) {
+      lds_ptr<float> out = part_slot<REGS>(smem, wave - RW, lane);
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[(16 * db + r) * 64] = acc[db][r];
+      if constexpr (MODE == 0) {
+        out[16 * DB * 64] = m_run;
+        out[(16 * DB + 1) * 64] = l_run;
+      }
+    }
+    __syncthreads();
+    if (sub > 0) return;
+    // a wave that saw no key has m = -1e30, l = 0 and weighs nothing
+#pragma unroll
+    for (int w = 0; w < SPLIT - 1; ++w) {
+      lds_ptr<float> in = part_slot<REGS>(smem, w * RW + wave, lane);
+      float a0 = 1.0f, a1 = 1.0f;
+      if constexpr (MODE == 0) {
+        const float m1 = in[16 * DB * 64];
+        const float mn = fmaxf(m_run, m1);
+        a0 = fast_exp2(m_run - mn);
+        a1 = fast_exp2(m1 - mn);
+        m_run = mn;
+        l_run = l_run * a0 + in[(16 * DB + 1) * 64] * a1;
+      }
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[db][r] = MODE == 0 ? acc[db][r] * a0 + in[(16 * db + r) * 64] * a1 : acc[db][r] + in[(16 * db + r) * 64];
+    }
+  }
+
   // ---- store: lane's row, d = 32 db + 8 (r/4) + 4 hi + r%4 ----
   float mul;
   if constexpr (MODE == 0) {
@@ -627,34 +737,36 @@ __global__ __launch_bounds__(kThreads) void query_major_kernel(TrainParams p) {
       const int d0 = 32 * db + 8 * rr + 4 * hi;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (VEC || d0 + j < D) op[d0 + j] = static_cast<T>(acc[db][4 * rr + j] * mul);
+        if (ROWS == kRowFull || d0 + j < D) op[d0 + j] = static_cast<T>(acc[db][4 * rr + j] * mul);
     }
 }
 
 // ---------------------------------------------------------------------------
 // Key-major kernel for 32 keys per wave: PASS 0 = dV, 1 = dK, 2 = both.
 constexpr int kPassDV = 0, kPassDK = 1, kPassBoth = 2;
-template <typename T, int DP, bool VEC, int PASS>
-__global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
+template <typename T, int DP, int DC, int ROWS, int PASS, int SPLIT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && DP <= 64 ? 2 : 1))) void dkdv_kernel(TrainParams p) {
   constexpr bool DO_DV = PASS != kPassDK;
   constexpr bool DO_DK = PASS != kPassDV;
   typedef typename Elem<T>::frag F;
-  constexpr int KK = DP / 16;
-  constexpr int DB = DP / 32;
-  constexpr bool DMA = VEC && sizeof(T) == 2;
-  typedef TileRing<T, DP, DMA, true> Ring;
+  constexpr int KK = DC / 16;
+  constexpr int DB = (DC + 31) / 32;
+  constexpr bool DMA = ROWS != kRowElems && sizeof(T) == 2;
+  constexpr int RW = kWaves / SPLIT;  // 32-key blocks per workgroup
+  typedef TileRing<T, DP, DMA, true, kRows * SPLIT, ROWS> Ring;
   __shared__ __attribute__((aligned(1024))) char smem[Ring::BYTES];
 
   const int N = p.N, D = p.D;
   int bh, blk;
   if (!map_block(p, false, bh, blk)) return;
-  const int k0 = blk * kBlockRows;
+  const int k0 = blk * (RW * kRows);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int hi = lane >> 5;
-  const int wk0 = k0 + wave * kRows;
+  const int sub = wave / RW;  // sub-tile of each streamed tile this wave computes
+  const int wk0 = k0 + (wave % RW) * kRows;
   const int krow = wk0 + l32;
   const bool kvalid = krow < N;
   const size_t base = static_cast<size_t>(bh) * N * D;
@@ -669,8 +781,8 @@ __global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
     const T* vr = static_cast<const T*>(p.v) + base + static_cast<size_t>(min(krow, N - 1)) * D;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      kf[kk] = kvalid ? load_frag<T, VEC>(kr, 16 * kk + 8 * hi, D) : zero_frag<T>();
-      if constexpr (DO_DK) vf[kk] = kvalid ? load_frag<T, VEC>(vr, 16 * kk + 8 * hi, D) : zero_frag<T>();
+      kf[kk] = kvalid ? load_frag<T, ROWS>(kr, 16 * kk + 8 * hi, D) : zero_frag<T>();
+      if constexpr (DO_DK) vf[kk] = kvalid ? load_frag<T, ROWS>(vr, 16 * kk + 8 * hi, D) : zero_frag<T>();
     }
   }
   float16_t dk[DB], dv[DB];
@@ -685,22 +797,26 @@ __global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
 
   // query tiles this workgroup needs: causal skips rows before its first key
   const int qstart = p.causal ? k0 : 0;
-  const int ntiles = (N - qstart + kRows - 1) / kRows;
+  constexpr int SR = Ring::SR;
+  const int ntiles = (N - qstart + SR - 1) / SR;
 
   Ring ring(smem, tid, D);
   const Reader<T, DP> rd(lane);
-  // a tile whose last query precedes this wave's first key contributes nothing:
-  // causal waves start at the tile holding query wk0
-  const int c_begin = wk0 >= N ? ntiles : (p.causal ? (wk0 - qstart) / kRows : 0);  // no keys: no compute
+  constexpr unsigned kSubBytes = kRows * Layout<T, DP>::LD * sizeof(T);
+  // a sub-tile whose last query precedes this wave's first key contributes
+  // nothing: causal waves start at the tile whose sub-tile holds or follows
+  // query wk0; sub-tiles past the last query are not computed either
+  const int c_begin = wk0 >= N ? ntiles : (p.causal ? max(0, wk0 - qstart - sub * kRows + SR - kRows) / SR : 0);
+  const int c_end = (N - qstart - sub * kRows + SR - 1) / SR;
   // (the register-staged fp32 pass measured no gain from it)
   // The dV pass never reads delta, and runs concurrently with the kernel that
   // writes it: its second per-row stream is pointed at lse instead (staged,
   // never used), so it touches nothing that kernel writes.
   const float* __restrict__ vb_rows = DO_DK ? dlt : lse;
-  run_ring<Ring, DMA, VEC, FA_BWD_REV != 0 && DMA>(ring, qp, dop, lse, vb_rows, qstart, ntiles, c_begin, ntiles, N, D, [&](int stage, int t) {
-    const int qt = qstart + t * kRows;
-    const unsigned qs = ring.addr_a(stage);
-    const unsigned ds = ring.addr_b(stage);
+  run_ring<Ring, DMA, FA_BWD_REV != 0 && DMA>(ring, qp, dop, lse, vb_rows, qstart, ntiles, c_begin, c_end, N, D, [&](int stage, int t) {
+    const int qt = qstart + t * SR + sub * kRows;
+    const unsigned qs = ring.addr_a(stage) + sub * kSubBytes;
+    const unsigned ds = ring.addr_b(stage) + sub * kSubBytes;
     // S = Q K^T and dP = dO V^T: lane <-> key, register r <-> query qt + 8 (r/4) + 4 hi + r%4
     float16_t s, dp;
 #pragma unroll
@@ -719,8 +835,8 @@ __global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
     const bool diag = p.causal && qt < wk0 + kRows - 1;
     const int lo = diag ? qt + 4 * hi - krow : 0;
     const int lim = tail ? N - qt - 4 * hi : kRows;
-    const __attribute__((address_space(3))) float* lv = ring.vec(stage, 0);
-    const __attribute__((address_space(3))) float* dvv = ring.vec(stage, 1);
+    const __attribute__((address_space(3))) float* lv = ring.vec(stage, 0) + sub * kRows;
+    const __attribute__((address_space(3))) float* dvv = ring.vec(stage, 1) + sub * kRows;
     const float lmul = DMA ? kLog2e : 1.0f;  // the register path stores lse pre-scaled
     const bool need_mask = tail || diag;  // wave-uniform: diagonal or last tile only
     float16_t pm, dsm;
@@ -765,6 +881,36 @@ __global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
     }
   });
 
+  // ---- join the key block's waves: wave `sub` 0 takes the others' partials ----
+  if constexpr (SPLIT > 1) {
+    constexpr int REGS = 16 * DB;
+    static_assert((SPLIT - 1) * RW * REGS * 256 <= Ring::BYTES, "partials fit the ring");
+    auto join = [&](float16_t (&x)[DB]) {
+      __syncthreads();  // every wave is done reading the ring (or the previous partials)
+      if (sub > 0) {
+        lds_ptr<float> out = part_slot<REGS>(smem, wave - RW, lane);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) out[(16 * db + r) * 64] = x[db][r];
+      }
+      __syncthreads();
+      if (sub == 0) {
+#pragma unroll
+        for (int w = 0; w < SPLIT - 1; ++w) {
+          lds_ptr<float> in = part_slot<REGS>(smem, w * RW + wave, lane);
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x[db][r] += in[(16 * db + r) * 64];
+        }
+      }
+    };
+    if constexpr (DO_DV) join(dv);
+    if constexpr (DO_DK) join(dk);
+    if (sub > 0) return;
+  }
+
   if (!kvalid) return;
   T* dkp = static_cast<T*>(p.dk) + base + static_cast<size_t>(krow) * D;
   T* dvp = static_cast<T*>(p.dv) + base + static_cast<size_t>(krow) * D;
@@ -775,7 +921,7 @@ __global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
       const int d0 = 32 * db + 8 * rr + 4 * hi;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (VEC || d0 + j < D) {
+        if (ROWS == kRowFull || d0 + j < D) {
           if constexpr (DO_DK) dkp[d0 + j] = static_cast<T>(dk[db][4 * rr + j] * p.scale);
           if constexpr (DO_DV) dvp[d0 + j] = static_cast<T>(dv[db][4 * rr + j]);
         }
@@ -786,7 +932,7 @@ __global__ __launch_bounds__(kThreads) void dkdv_kernel(TrainParams p) {
 // query-major kernel's exact arithmetic: two fma chains per row, over
 // d = 16 kk + 8 h + j (h = 0, 1; kk = 0 .. DP/16 - 1; j = 0 .. 7; zero past D),
 // then their sum.  Two threads per row.
-template <typename T, int DP, bool VEC>
+template <typename T, int DP, int ROWS>
 __global__ __launch_bounds__(256) void delta_kernel(TrainParams p) {
   typedef typename Elem<T>::frag F;
   const long long t = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
@@ -798,8 +944,8 @@ __global__ __launch_bounds__(256) void delta_kernel(TrainParams p) {
   float part = 0.0f;
 #pragma unroll
   for (int kk = 0; kk < DP / 16; ++kk) {
-    const F df = load_frag<T, VEC>(dr, 16 * kk + 8 * h, p.D);
-    const F of = load_frag<T, VEC>(orow, 16 * kk + 8 * h, p.D);
+    const F df = load_frag<T, ROWS>(dr, 16 * kk + 8 * h, p.D);
+    const F of = load_frag<T, ROWS>(orow, 16 * kk + 8 * h, p.D);
 #pragma unroll
     for (int j = 0; j < 8; ++j) part = fmaf(static_cast<float>(df[j]), static_cast<float>(of[j]), part);
   }
@@ -821,15 +967,48 @@ hipStream_t backward_side_stream(hipStream_t caller, int which);
 // cannot be made.
 bool backward_events(hipEvent_t (&ev)[4]);
 
-template <typename T, int DP, bool VEC>
-void launch_backward_dp(const TrainParams& p, hipStream_t st) {
+// How a backward call runs, from the number of 128-row blocks it has (us of a
+// causal call, heavy-first single-wave blocks forked onto side streams -> the
+// rule's choice; all on one box):
+//  * fp16, up to 512 blocks: split in two, in order on the caller's stream (the
+//    fork and its events cost the host 30 us): [1,8,128,128] 61 -> 32,
+//    [2,16,512,128] 61 -> 43, [1,8,2048,128] 160 -> 109, [2,16,1000,64] 66 -> 47.
+//  * fp16, more: unsplit; D > 64 forked, dQ as a snake ([4,16,2048,128] 316, heavy
+//    first 320, in order 336, split 370), D <= 64 in order ([4,16,2048,64] 187 -> 167).
+//  * fp32 D <= 64: in order; split up to 512 blocks ([2,16,1000,64] 259 -> 183,
+//    [1,8,2048,64] 582 -> 381; [4,16,2048,64] 1193 -> 1054 unsplit).
+//  * fp32 D > 64: forked; up to 128 blocks split and dQ's blocks light first,
+//    against dK/dV's heavy first on the same CUs ([1,8,2048,128] 1110 -> 870,
+//    [2,16,512,128] 181 -> 121; [2,16,1000,128] 349 either way).
+struct BackwardPlan {
+  int split;
+  bool fork;
+  BlockOrder dq, dkdv;
+};
+template <typename T, int DP>
+BackwardPlan backward_plan(const TrainParams& p) {
+  const long long blocks = static_cast<long long>(p.BH) * ceil_div(p.N, kBlockRows);
+  if (sizeof(T) == 4 && DP > 64)
+    return blocks <= 128 ? BackwardPlan{2, true, kLightFirst, kHeavyFirst} : BackwardPlan{1, true, kHeavyFirst, kHeavyFirst};
+  if (blocks <= 512) return BackwardPlan{2, false, kSnake, kSnake};
+  if (sizeof(T) == 4) return BackwardPlan{1, false, kHeavyFirst, kHeavyFirst};
+  if (DP > 64) return BackwardPlan{1, true, kSnake, kHeavyFirst};
+  return BackwardPlan{1, false, kSnake, kSnake};
+}
+
+template <typename T, int DP, int DC, int ROWS, int SPLIT>
+void launch_backward_split(TrainParams p, const BackwardPlan& plan, hipStream_t st) {
+  p.nblk = ceil_div(p.N, kBlockRows / SPLIT);
+  p.order = plan.dkdv;
+  TrainParams pq = p;
+  pq.order = plan.dq;
   const dim3 grid(train_grid(p));
   // fp16 at D > 64 splits dV and dK into two passes to fit 256 VGPRs
 #ifndef FA_BWD_SPLIT_DKDV
 #define FA_BWD_SPLIT_DKDV 1
 #endif
   constexpr bool kSplit = FA_BWD_SPLIT_DKDV && sizeof(T) == 2 && DP > 64;
-  {
+  if (plan.fork) {
     // Concurrent streams: delta (a short kernel) then dQ on `st`; the dK/dV
     // pass (or the dK pass) on a side stream once delta is there; with split
     // passes, the dV pass, which needs neither, on another side stream from
@@ -847,21 +1026,20 @@ void launch_backward_dp(const TrainParams& p, hipStream_t st) {
     if (ok) {
       bool v_joined = true;
       if constexpr (kSplit) {
-        hipLaunchKernelGGL((dkdv_kernel<T, DP, VEC, kPassDV>), grid, dim3(kThreads), 0, side_v, p);
+        hipLaunchKernelGGL((dkdv_kernel<T, DP, DC, ROWS, kPassDV, SPLIT>), grid, dim3(kThreads), 0, side_v, p);
         v_joined = hipEventRecord(ev[2], side_v) == hipSuccess;
       }
       const long long rows = static_cast<long long>(p.BH) * p.N;
-      hipLaunchKernelGGL((delta_kernel<T, DP, VEC>), dim3(static_cast<unsigned>((2 * rows + 255) / 256)), dim3(256), 0,
+      hipLaunchKernelGGL((delta_kernel<T, DP, ROWS>), dim3(static_cast<unsigned>((2 * rows + 255) / 256)), dim3(256), 0,
                          st, p);
-      TrainParams pq = p;
       pq.delta_ready = 1;
       const bool k_forked = hipEventRecord(ev[1], st) == hipSuccess && hipStreamWaitEvent(side_k, ev[1], 0) == hipSuccess;
-      hipLaunchKernelGGL((query_major_kernel<T, DP, VEC, 1>), grid, dim3(kThreads), 0, st, pq);
+      hipLaunchKernelGGL((query_major_kernel<T, DP, DC, ROWS, 1, SPLIT>), grid, dim3(kThreads), 0, st, pq);
       hipStream_t sk = k_forked ? side_k : st;
       if constexpr (kSplit)
-        hipLaunchKernelGGL((dkdv_kernel<T, DP, VEC, kPassDK>), grid, dim3(kThreads), 0, sk, p);
+        hipLaunchKernelGGL((dkdv_kernel<T, DP, DC, ROWS, kPassDK, SPLIT>), grid, dim3(kThreads), 0, sk, p);
       else
-        hipLaunchKernelGGL((dkdv_kernel<T, DP, VEC, kPassBoth>), grid, dim3(kThreads), 0, sk, p);
+        hipLaunchKernelGGL((dkdv_kernel<T, DP, DC, ROWS, kPassBoth, SPLIT>), grid, dim3(kThreads), 0, sk, p);
       // joins; should one fail, wait for that stream on the host instead
       if (k_forked && (hipEventRecord(ev[3], side_k) != hipSuccess || hipStreamWaitEvent(st, ev[3], 0) != hipSuccess))
         (void)hipStreamSynchronize(side_k);
@@ -870,47 +1048,94 @@ void launch_backward_dp(const TrainParams& p, hipStream_t st) {
     }
     (void)hipGetLastError();  // a failed fork leaves no error behind: run in order below
   }
-  hipLaunchKernelGGL((query_major_kernel<T, DP, VEC, 1>), grid, dim3(kThreads), 0, st, p);
+  hipLaunchKernelGGL((query_major_kernel<T, DP, DC, ROWS, 1, SPLIT>), grid, dim3(kThreads), 0, st, pq);
   if constexpr (kSplit) {
-    hipLaunchKernelGGL((dkdv_kernel<T, DP, VEC, kPassDV>), grid, dim3(kThreads), 0, st, p);
-    hipLaunchKernelGGL((dkdv_kernel<T, DP, VEC, kPassDK>), grid, dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL((dkdv_kernel<T, DP, DC, ROWS, kPassDV, SPLIT>), grid, dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL((dkdv_kernel<T, DP, DC, ROWS, kPassDK, SPLIT>), grid, dim3(kThreads), 0, st, p);
   } else {
-    hipLaunchKernelGGL((dkdv_kernel<T, DP, VEC, kPassBoth>), grid, dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL((dkdv_kernel<T, DP, DC, ROWS, kPassBoth, SPLIT>), grid, dim3(kThreads), 0, st, p);
   }
 }
 
-// dQ (+ delta) then dK/dV for any 1 <= D <= 128.  fp16 tiles need DP >= 64
-// (the swizzle covers 8 or 16 chunks per row), so D <= 64 runs at DP = 64.
+template <typename T, int DP, int DC, int ROWS>
+void launch_backward_dp(const TrainParams& p, hipStream_t st) {
+  if constexpr (ROWS != kRowElems) {
+    const BackwardPlan plan = backward_plan<T, DP>(p);
+    if (plan.split == 2) launch_backward_split<T, DP, DC, ROWS, 2>(p, plan, st);
+    else launch_backward_split<T, DP, DC, ROWS, 1>(p, plan, st);
+  } else {
+    launch_backward_split<T, DP, DC, ROWS, 1>(p, BackwardPlan{1, true, kHeavyFirst, kHeavyFirst}, st);
+  }
+}
+
+// dQ (+ delta) then dK/dV for any 1 <= D <= 128.  fp16 tiles need DP of 64 or
+// 128 (the swizzle covers 8 or 16 chunks per row); their products stop at the
+// narrowest built DC that holds D.
 template <typename T>
-void launch_backward(const TrainParams& p, bool vec_ok, hipStream_t st) {
+void launch_backward(const TrainParams& p, bool aligned, hipStream_t st) {
   const int D = p.D;
+  const bool vec = aligned && D % 8 == 0;
   if constexpr (sizeof(T) == 4) {
-    if (D <= 32) {
-      vec_ok && D == 32 ? launch_backward_dp<T, 32, true>(p, st) : launch_backward_dp<T, 32, false>(p, st);
+    if (!vec) {
+      if (D <= 32) launch_backward_dp<T, 32, 32, kRowElems>(p, st);
+      else if (D <= 64) launch_backward_dp<T, 64, 64, kRowElems>(p, st);
+      else launch_backward_dp<T, 128, 128, kRowElems>(p, st);
+    } else if (D <= 32) launch_backward_dp<T, 32, 32, kRowChunks>(p, st);
+    else if (D == 64) launch_backward_dp<T, 64, 64, kRowFull>(p, st);
+    else if (D < 64) launch_backward_dp<T, 64, 64, kRowChunks>(p, st);
+    else if (D <= 96) launch_backward_dp<T, 96, 96, kRowChunks>(p, st);
+    else if (D == 128) launch_backward_dp<T, 128, 128, kRowFull>(p, st);
+    else launch_backward_dp<T, 128, 128, kRowChunks>(p, st);
+  } else {
+    if (!vec) {
+      if (D <= 64) launch_backward_dp<T, 64, 64, kRowElems>(p, st);
+      else launch_backward_dp<T, 128, 128, kRowElems>(p, st);
+    } else if (D == 64) launch_backward_dp<T, 64, 64, kRowFull>(p, st);
+    else if (D < 64) launch_backward_dp<T, 64, 64, kRowChunks>(p, st);
+    else if (D <= 96) launch_backward_dp<T, 128, 96, kRowChunks>(p, st);
+    else if (D == 128) launch_backward_dp<T, 128, 128, kRowFull>(p, st);
+    else launch_backward_dp<T, 128, 128, kRowChunks>(p, st);
+  }
+}
+
+template <int DP, int ROWS, int SPLIT>
+void launch_forward_split(TrainParams p, hipStream_t st) {
+  p.nblk = ceil_div(p.N, kBlockRows / SPLIT);
+  p.order = kSnake;
+  hipLaunchKernelGGL((query_major_kernel<float, DP, DP, ROWS, 0, SPLIT>), dim3(train_grid(p)), dim3(kThreads), 0, st, p);
+}
+
+// The fp32 forward splits its blocks in two at D <= 64 at every size measured
+// (causal [2,16,1000,64] 82 -> 49 us, [1,8,2048,64] 216 -> 114, [4,16,2048,64]
+// 346 -> 322; full [2,16,1024,64] 81 -> 79), and at D > 64, where a split
+// workgroup's two stages take most of a CU's LDS, only grids that leave CUs idle
+// or a lone causal workgroup on each ([2,16,512,128] 77 -> 46, [2,16,1000,128]
+// 151 -> 96-119; full [2,16,1024,128] 155 unsplit, 171 split).
+template <int DP, int ROWS>
+void launch_forward_dp(const TrainParams& p, hipStream_t st) {
+  if constexpr (ROWS != kRowElems) {
+    const long long blocks = static_cast<long long>(p.BH) * ceil_div(p.N, kBlockRows);
+    if (DP <= 64 || blocks <= (p.causal ? 256 : 128)) {
+      launch_forward_split<DP, ROWS, 2>(p, st);
       return;
     }
   }
-  if (D <= 64) {
-    vec_ok && D == 64 ? launch_backward_dp<T, 64, true>(p, st) : launch_backward_dp<T, 64, false>(p, st);
-  } else {
-    vec_ok && D == 128 ? launch_backward_dp<T, 128, true>(p, st) : launch_backward_dp<T, 128, false>(p, st);
-  }
+  launch_forward_split<DP, ROWS, 1>(p, st);
 }
 
 // fp32 forward (O and optional log-sum-exp) for any 1 <= D <= 128.
-inline void launch_forward_fp32(const TrainParams& p, bool vec_ok, hipStream_t st) {
+inline void launch_forward_fp32(const TrainParams& p, bool aligned, hipStream_t st) {
   const int D = p.D;
-  const dim3 grid(train_grid(p));
-  if (D <= 32) {
-    if (vec_ok && D == 32) hipLaunchKernelGGL((query_major_kernel<float, 32, true, 0>), grid, dim3(kThreads), 0, st, p);
-    else hipLaunchKernelGGL((query_major_kernel<float, 32, false, 0>), grid, dim3(kThreads), 0, st, p);
-  } else if (D <= 64) {
-    if (vec_ok && D == 64) hipLaunchKernelGGL((query_major_kernel<float, 64, true, 0>), grid, dim3(kThreads), 0, st, p);
-    else hipLaunchKernelGGL((query_major_kernel<float, 64, false, 0>), grid, dim3(kThreads), 0, st, p);
-  } else {
-    if (vec_ok && D == 128) hipLaunchKernelGGL((query_major_kernel<float, 128, true, 0>), grid, dim3(kThreads), 0, st, p);
-    else hipLaunchKernelGGL((query_major_kernel<float, 128, false, 0>), grid, dim3(kThreads), 0, st, p);
-  }
+  if (!aligned || D % 8 != 0) {
+    if (D <= 32) launch_forward_dp<32, kRowElems>(p, st);
+    else if (D <= 64) launch_forward_dp<64, kRowElems>(p, st);
+    else launch_forward_dp<128, kRowElems>(p, st);
+  } else if (D <= 32) launch_forward_dp<32, kRowChunks>(p, st);
+  else if (D == 64) launch_forward_dp<64, kRowFull>(p, st);
+  else if (D < 64) launch_forward_dp<64, kRowChunks>(p, st);
+  else if (D <= 96) launch_forward_dp<96, kRowChunks>(p, st);
+  else if (D == 128) launch_forward_dp<128, kRowFull>(p, st);
+  else launch_forward_dp<128, kRowChunks>(p, st);
 }
 
 // Entry point of the fp32 backward translation unit (train_fp32.hip).

@@ -174,3 +174,73 @@ def test_decode_chunk_rows_special_values(fa, d, b, hq, hkv, n):
     assert equal(fa.forward_decode_gqa_fp16(q, k, v, True, n - 1), fa.forward_decode_gqa_fp16(qm, k, v, True, n - 1))
     assert equal(fa.forward_continuous_batching_fp16(q, k, v, lens, True),
                  fa.forward_continuous_batching_fp16(qm, k, v, lens, True))
+
+
+def _grads_close(got, ref, fp16):
+    """fp16: 3e-2 + 3e-2 |x| and rel-L2 1e-2, fp32: 2e-4 + 2e-4 |x| (the bounds of
+    the training tests)."""
+    tol = 3e-2 if fp16 else 2e-4
+    for name, a, r in zip(("dq", "dk", "dv"), got, ref):
+        assert_close(a, r, atol=tol, rtol=tol, what=name)
+        if fp16 and r.double().norm() > 1e-3:
+            assert (a.double().cpu() - r.double().cpu()).norm() <= 1e-2 * r.double().cpu().norm(), name
+
+
+def _train(fa, q, k, v, do, causal):
+    fwd = fa.forward_fp16_with_lse if q.dtype == torch.float16 else fa.forward_with_lse
+    out, lse = fwd(q, k, v, causal)
+    return out, lse, fa.backward(do, q, k, v, out, lse, causal)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("b,h,n,d", [
+    (1, 9, 1, 80), (1, 9, 63, 72), (2, 4, 64, 96), (2, 5, 65, 40), (1, 8, 127, 120), (3, 3, 193, 24),
+    (1, 2, 130, 88), (2, 8, 385, 80),           # rows of whole chunks, split blocks
+    (1, 9, 31, 64), (2, 4, 97, 64), (1, 8, 129, 128), (2, 8, 450, 128)])  # edges of split 32-row sub-tiles
+def test_training_chunk_rows_and_split_blocks(fa, dtype, causal, b, h, n, d):
+    g = gen(n * 31 + d)
+    q, k, v, do = (randn(g, b, h, n, d, dtype=dtype) for _ in range(4))
+    out, lse, grads = _train(fa, *(t.to(DEV) for t in (q, k, v, do)), causal)
+    ro, rl = A.prefill_lse(q, k, v, causal, compute_dtype=torch.float64)
+    fp16 = dtype == torch.float16
+    assert_close(out, ro, **({} if fp16 else {"atol": 2e-4, "rtol": 2e-4}), what="out")
+    assert_close(lse, rl, atol=2e-3 if fp16 else 2e-4, rtol=0 if fp16 else 2e-4, what="lse")
+    _grads_close(grads, A.backward(do, q, k, v, out.cpu(), lse.cpu(), causal), fp16)
+    again = _train(fa, *(t.to(DEV) for t in (q, k, v, do)), causal)[2]
+    assert all(torch.equal(x, y) for x, y in zip(grads, again))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("d", [64, 80, 128])
+def test_training_large_grid_matches_its_parts(fa, dtype, d):
+    """A call past the grid size up to which blocks are split (512 blocks of 128
+    rows) agrees with the same heads in a small, split call."""
+    g = gen(d)
+    q, k, v, do = (randn(g, 8, 13, 580, d, dtype=dtype).to(DEV) for _ in range(4))  # 520 blocks
+    big = _train(fa, q, k, v, do, True)
+    part = _train(fa, *(t[3:5].contiguous() for t in (q, k, v, do)), True)
+    fp16 = dtype == torch.float16
+    tol = {} if fp16 else {"atol": 2e-4, "rtol": 2e-4}
+    assert_close(big[0][3:5], part[0], **tol, what="out")
+    assert_close(big[1][3:5], part[1], atol=2e-3 if fp16 else 2e-4, rtol=0, what="lse")
+    _grads_close([x[3:5] for x in big[2]], part[2], fp16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_training_in_order_calls_capture(fa, dtype):
+    """A small backward under graph capture equals the eager one on every replay."""
+    g = gen(5)
+    q, k, v, do = (randn(g, 1, 8, 200, 80, dtype=dtype).to(DEV) for _ in range(4))
+    out, lse, ref = _train(fa, q, k, v, do, True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = fa.backward(do, q, k, v, out, lse, True)
+    for _ in range(3):
+        for x in got:
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, ref))
+        _train(fa, q, k, v, do, False)
