@@ -113,22 +113,22 @@ struct PrefillParams {
 // ring has 4 stages, so three tiles are in flight from the start (short
 // sequences: most of the keys).
 //
-// KSPLIT (D <= 128, launches far smaller than the chip): the four waves share
-// one 32-row query block and split every 128-key tile, wave w taking keys
-// 32w .. 32w + 31; their partial (max, sum, O) merge through LDS at the end.
-// Each wave's serial chain is then a quarter of the keys, which is what bounds
-// short prefills that occupy only a few dozen CUs.
-template <int DP, bool WIDE = false, bool KSPLIT = false, int DC = DP>
+// KS > 1 (launches too small to hide a wave's serial chain of tiles behind
+// other waves): KS waves share one 32-row query block (4 / KS blocks per
+// workgroup) and split every 32 KS-key tile, wave w taking the 32 keys of
+// sub-tile w / (4 / KS); their partial (max, sum, O) merge through LDS at the
+// end.  Each wave's chain is then 1 / KS of the keys.
+template <int DP, bool WIDE = false, int KS = 1, int DC = DP>
 struct PrefillShape {
-  static constexpr int RB = KSPLIT ? 1 : (DP <= 64 ? FA_PRE_RB64 : 1);  // 32-row query blocks per wave
+  static constexpr int RB = KS > 1 ? 1 : (DP <= 64 ? FA_PRE_RB64 : 1);  // 32-row query blocks per wave
   static constexpr int RW = 32 * RB;                                    // query rows per wave
-  static constexpr int BQ = KSPLIT ? RW : kPreWaves * RW;               // query rows per workgroup
-  static constexpr int BK = KSPLIT ? 32 * kPreWaves : (DP <= 64 ? (WIDE ? 64 : FA_PRE_BK64) : 32);  // keys per tile
-  static constexpr int NS = KSPLIT ? (DP <= 64 ? 3 : 2)
+  static constexpr int BQ = kPreWaves / KS * RW;                        // query rows per workgroup
+  static constexpr int BK = KS > 1 ? 32 * KS : (DP <= 64 ? (WIDE ? 64 : FA_PRE_BK64) : 32);  // keys per tile
+  static constexpr int NS = KS > 1 ? (DP <= 64 ? 3 : 2)
                                    : (DP <= 64 ? (WIDE ? FA_PRE_NSW : 3) : (DP <= 128 ? FA_PRE_NS128 : 2));  // LDS ring stages
   static constexpr int TILE = BK * DP;                                  // halves per K (or V) tile
   static constexpr int WAVES_PER_SIMD =
-      KSPLIT ? 2 : (DP <= 64 ? (WIDE ? 3 : FA_PRE_W64) : (DP <= 128 ? (DC <= 96 ? 4 : FA_PRE_W128) : 2));  // register budget target
+      KS > 1 ? 2 : (DP <= 64 ? (WIDE ? 3 : FA_PRE_W64) : (DP <= 128 ? (DC <= 96 ? 4 : FA_PRE_W128) : 2));  // register budget target
 };
 
 // Varlen output rows that no sequence's attention writes are set to zero by
@@ -171,10 +171,10 @@ __device__ __forceinline__ void preload_args(const PrefillParams& p) {
 }
 
 // DP: padded row width in LDS; DC: columns computed (D <= DC <= DP).
-template <int DP, int DC, bool VARLEN, int ROWS, bool WIDE = false, bool KSPLIT = false>
+template <int DP, int DC, bool VARLEN, int ROWS, bool WIDE = false, int KS = 1>
 __global__ __launch_bounds__(kPreThreads)
-__attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER_SIMD))) void prefill_kernel(PrefillParams p) {
-  using Shape = PrefillShape<DP, WIDE, KSPLIT, DC>;
+__attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIMD))) void prefill_kernel(PrefillParams p) {
+  using Shape = PrefillShape<DP, WIDE, KS, DC>;
   constexpr bool VEC = ROWS != kRowElems;
   constexpr int RB = Shape::RB;
   constexpr int RW = Shape::RW;
@@ -182,7 +182,8 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER
   constexpr int kBK = Shape::BK;
   constexpr int NS = Shape::NS;
   constexpr int TILE = Shape::TILE;
-  constexpr int NBLK = KSPLIT ? 1 : kBK / 32;  // 32-key blocks per tile computed by one wave
+  constexpr int RG = kPreWaves / KS;          // query blocks per workgroup
+  constexpr int NBLK = KS > 1 ? 1 : kBK / 32;  // 32-key blocks per tile computed by one wave
   constexpr int KK = DC / 16;                 // 16-wide d slices of QK^T
   constexpr int DB = (DC + 31) / 32;          // 32-row d blocks of PV
   constexpr int CPR = DP / 8;                 // 16-byte chunks per row
@@ -261,8 +262,8 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int hi = lane >> 5;
-  const int wq0 = q0 + (KSPLIT ? 0 : wave * RW);  // first query row of this wave
-  const int kw = KSPLIT ? 32 * wave : 0;            // first key of this wave's block inside a tile
+  const int wq0 = q0 + wave % RG * RW;  // first query row of this wave
+  const int kw = 32 * (wave / RG);      // first key of this wave's block inside a tile (0 unless split)
 
   const half_t* __restrict__ qp = p.q + q_base;
   const half_t* __restrict__ kp = p.k + k_base;
@@ -513,12 +514,12 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER
     tile_barrier();  // every wave's copies of tile t landed; stage (t-1) % NS is free
     if (t + NS - 1 < ntiles) issue(t + NS - 1);
     const int kt = t * kBK + kw;
-    constexpr int kWaveKeys = KSPLIT ? 32 : kBK;  // keys of a tile this wave computes
+    constexpr int kWaveKeys = KS > 1 ? 32 : kBK;  // keys of a tile this wave computes
     if (kt >= kend_w) continue;  // past this wave's diagonal (still copies and joins the barriers)
     compute_tile(t, (kt + kWaveKeys > seq_len) || (p.causal && kt + kWaveKeys - 1 > wq0));
   }
 
-  if constexpr (KSPLIT) {
+  if constexpr (KS == 4) {
     // ---- merge the four waves' partials of the shared 32 rows ----
     // Lane (l32, hi) holds O[l32][32 db + 8 rr + 4 hi + j] = oacc[db][0][4 rr + j]
     // against its wave's max m; scaled to the common max M, the waves' O and
@@ -591,6 +592,36 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER
     return;
   }
 
+  if constexpr (KS == 2) {
+    // ---- merge the two waves of each query block: both hold an element in the
+    // same lane and register, so the second wave's partials pass lane to lane
+    constexpr int REGS = 16 * DB + 2;
+    static_assert(RG * REGS * 256 <= NS * 2 * TILE * 2, "partials fit the ring");
+    auto* part = reinterpret_cast<__attribute__((address_space(3))) float*>(static_cast<size_t>(lds_base)) +
+                 wave % RG * REGS * 64 + lane;
+    __syncthreads();  // every wave is done reading the ring
+    if (kw != 0) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[(16 * db + r) * 64] = oacc[db][0][r];
+      part[16 * DB * 64] = m_run[0];
+      part[(16 * DB + 1) * 64] = l_run[0];
+    }
+    __syncthreads();
+    if (kw != 0) return;
+    // (a wave that saw no key has m = -1e30, l = 0 and weighs nothing)
+    const float m1 = part[16 * DB * 64];
+    const float mx = fmaxf(m_run[0], m1);
+    const float a0 = fast_exp2(m_run[0] - mx), a1 = fast_exp2(m1 - mx);
+    m_run[0] = mx;
+    l_run[0] = l_run[0] * a0 + part[(16 * DB + 1) * 64] * a1;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[db][0][r] = oacc[db][0][r] * a0 + part[(16 * db + r) * 64] * a1;
+  }
+
   // ---- finalize and store O[qrow][d] ----
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
@@ -626,12 +657,16 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KSPLIT, DC>::WAVES_PER
 }
 
 template <int DP, int DC, bool VARLEN, int ROWS>
-static void launch_shape(bool wide, bool ksplit, int blocks, const PrefillParams& p, hipStream_t st) {
+static void launch_shape(bool wide, int ks, int blocks, const PrefillParams& p, hipStream_t st) {
   if constexpr (DP <= 128) {
-    if (ksplit) {
-      hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS, false, true>), dim3(blocks), dim3(kPreThreads), 0, st, p);
+    if (ks == 4) {
+      hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS, false, 4>), dim3(blocks), dim3(kPreThreads), 0, st, p);
       return;
     }
+  }
+  if (ks == 2) {
+    hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS, false, 2>), dim3(blocks), dim3(kPreThreads), 0, st, p);
+    return;
   }
   if constexpr (DP <= 64) {
     if (wide) {
@@ -642,12 +677,8 @@ static void launch_shape(bool wide, bool ksplit, int blocks, const PrefillParams
   hipLaunchKernelGGL((prefill_kernel<DP, DC, VARLEN, ROWS>), dim3(blocks), dim3(kPreThreads), 0, st, p);
 }
 constexpr long long kWideMaxBlocks = 1024;  // D <= 64 launches up to this size use 64-key tiles
-// D <= 128 launches of at most this many 128-row workgroups run key-split
-// (four times as many 32-row workgroups).
-#ifndef FA_PRE_KSPLIT_MAX
-#define FA_PRE_KSPLIT_MAX 64
-#endif
-constexpr long long kKsplitMaxBlocks = FA_PRE_KSPLIT_MAX;
+constexpr long long kSplit4MaxBlocks = 64;   // see dispatch_prefill
+constexpr long long kSplit2MaxBlocks = 256;
 
 static int prefill_bq(int D) { return D <= 64 ? PrefillShape<64>::BQ : (D <= 128 ? PrefillShape<128>::BQ : PrefillShape<256>::BQ); }
 
@@ -655,8 +686,23 @@ static int prefill_bq(int D) { return D <= 64 ? PrefillShape<64>::BQ : (D <= 128
 // tail); returns FA_OK or an error code.
 template <bool VARLEN>
 static int dispatch_prefill(const char* fn, int D, bool vec, int rows_max, PrefillParams p, hipStream_t st) {
-  const bool ksplit = D <= 128 && static_cast<long long>(ceil_div(rows_max, prefill_bq(D))) * p.H_Q * p.B <= kKsplitMaxBlocks;
-  p.qtiles = ceil_div(rows_max, ksplit ? PrefillShape<64, false, true>::BQ : prefill_bq(D));
+  // Waves per query block, from the 128-row workgroups of an unsplit launch.
+  // A lone wave takes about 0.85 us a 32-key tile at D = 128, four times its
+  // MFMA time, so launches that leave SIMDs idle or with little to switch to
+  // are bound by the longest walk (causal unless noted, us unsplit -> split):
+  //   up to 64 (D <= 128): four waves ([2,8,512,64] 10.3 -> 6.7, two 8.1).
+  //   up to 256, causal up to 512 (D <= 128): two ([1,32:8,512,128] 16.8 -> 12.0,
+  //     four 13.5; [1,32:8,1024,128] 29.4 -> 20.6, four 34.8; full 31.0 -> 25.2;
+  //     [1,32:8,2048,128] 56.4 -> 49.7; [1,16,4096,64] 59.8 -> 49.8).
+  //   up to 256 at D > 128, where a split workgroup's LDS fills a CU: two
+  //     ([1,16,2048,256] 88 -> 69; 512 blocks 185 -> 239).
+  //   more: one, with three or more waves per SIMD ([1,32:8,4096,128], 1024
+  //     blocks, 145 -> 171 split; full [2,32:8,1024,128], 512 blocks, 42 -> 48).
+  const long long whole = static_cast<long long>(ceil_div(rows_max, prefill_bq(D))) * p.H_Q * p.B;
+  int ks = 1;
+  if (D <= 128 && whole <= kSplit4MaxBlocks) ks = 4;
+  else if (whole <= (D <= 128 && p.causal ? 2 * kSplit2MaxBlocks : kSplit2MaxBlocks)) ks = 2;
+  p.qtiles = ceil_div(rows_max, prefill_bq(D) / ks);
 #if FA_PRE_ORDER == 0
   const long long main_blocks = static_cast<long long>(p.qtiles) * p.H_Q * p.B;
 #else
@@ -679,7 +725,7 @@ static int dispatch_prefill(const char* fn, int D, bool vec, int rows_max, Prefi
   const bool wide = main_blocks <= kWideMaxBlocks;
   const int n = static_cast<int>(blocks);
   auto run = [&](auto dp, auto dc, auto mode) {
-    launch_shape<dp(), dc(), VARLEN, mode()>(wide, ksplit, n, p, st);
+    launch_shape<dp(), dc(), VARLEN, mode()>(wide, ks, n, p, st);
   };
   constexpr std::integral_constant<int, kRowElems> elems;
   constexpr std::integral_constant<int, kRowFull> full;

@@ -85,6 +85,22 @@ def test_prefill_chunk_rows_special_values(fa, d):
         assert not torch.isnan(out[0, 0]).any()
 
 
+@pytest.mark.parametrize("d", [64, 80, 128, 256])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("b,h,n", [(1, 32, 260), (3, 24, 129), (1, 70, 33), (2, 40, 321)])
+def test_prefill_two_wave_blocks(fa, d, causal, b, h, n):
+    """Launches whose query blocks are shared by two waves (65 to 256 or, causal,
+    512 blocks of 128 rows) at the edges of their 64-row and 64-key tiles."""
+    g = gen(d + n)
+    q, k, v = (randn(g, b, h, n, d) for _ in range(3))
+    out = fa.forward_fp16(*(t.to(DEV) for t in (q, k, v)), causal)
+    assert_close(out, A.prefill(q, k, v, causal), what=f"two-wave blocks {b, h, n, d}")
+    if d <= 128:
+        out2, lse = fa.forward_fp16_with_lse(*(t.to(DEV) for t in (q, k, v)), causal)
+        assert torch.equal(out, out2)
+        assert_close(lse, A.prefill_lse(q, k, v, causal)[1], atol=2e-3, rtol=0, what="lse")
+
+
 @pytest.mark.parametrize("d", [8, 32, 72, 80, 96, 112, 192, 200])
 @pytest.mark.parametrize("causal", [True, False])
 def test_varlen_chunk_rows(fa, d, causal):
