@@ -242,31 +242,36 @@ __global__ __launch_bounds__(kThreads) void evict_kernel(const half_t* __restric
 //
 // Those serial sums are computed in parallel, bit for bit.  While the running
 // sum s stays inside one binade it is n * g with g the ulp there and n an
-// integer, and adding a term t >= 0 moves n by an integer: rne(t / g), except
-// that an exact tie (t / g = k + 1/2) goes to the neighbour that makes n even.
-// A term is therefore a map from the parity of n to an increment, a pair
-// (d0, d1), and such pairs compose associatively: a wave scans the pairs of
-// its lanes' terms, a workgroup those of its waves.  A prefix is valid while
-// n <= 2^24; where it passes that (s leaves its binade), where a term is
-// negative or not finite, or where the comparison with r first holds, the
-// wave that owns the place walks it: it finds the first such lane by the same
-// scan, adds that lane's terms in fp32 one by one, and goes on from the sum it
-// gets.  A row of a thousand or more terms doubles its sum only a few times,
-// so nearly all of them go through the scans.
+// integer, and adding a term t >= 0 moves n by an integer that depends on t
+// and, where t / g is a tie, on the parity of n alone.  A run of terms is
+// therefore a map from the parity of n to an increment, a pair (d0, d1), found
+// by adding the terms in fp32 to any sum of that binade with n even and to one
+// with n odd; such pairs compose associatively, so lanes' pairs are scanned.
+// Which binade a lane's terms meet is told by an estimate of the sums (a float
+// prefix sum); a lane whose terms may cross into the next one is doubtful, and
+// its terms are added one by one.  One wave puts the pieces together with the
+// exact sum, and checks each piece against it: a wrong guess, a negative or
+// non-finite term or a hit sends that 512-term chunk to a walk, which locates
+// the lane concerned by the same scans and adds its terms in turn.  Only the
+// first chunk, where the sum doubles every few terms, is added serially.
 //
-// Bound by the latency of those passes (about 1.5 us a tile of 8192 terms, a
-// few more per row for the binades), not by bytes: a row of 32000 is read at
-// the rate one CU can pull.  Two workgroups per row run concurrently: Z, then
-// the residual sample; the bonus token.  One lane adding all the terms in turn
-// from LDS, fed by a second wave, took 180 us for 16 rows of 32000 words
-// and K = 4; this takes 63 us.
+// Bound by the latency of these steps, about 7 us a row of 32000 (2 us its
+// first chunk, 2 us the assembly), not by bytes.  Two workgroups per row run
+// concurrently: Z, then the residual sample; the bonus token.  One lane adding
+// all the terms in turn from LDS, fed by a second wave, took 180 us for 16 rows
+// of 32000 words and K = 4; scans that restarted at each binade 63 us; this
+// takes FIG_AFTER us.
 namespace spec {
 
 constexpr int kMaxK = 8;      // SPEC_MAX_K (flash_attn_kernel.cu:3851)
 constexpr int kWaves = 16;
 constexpr int kSpecThreads = kWaves * 64;
-constexpr int kTerms = 8;     // consecutive terms per thread and tile
-constexpr int kTile = kSpecThreads * kTerms;
+constexpr int kTerms = 8;               // consecutive terms per lane
+constexpr int kChunk = 64 * kTerms;     // consecutive terms per wave
+constexpr int kTiles = 4;               // chunks per wave and group
+constexpr int kChunks = kTiles * kWaves;  // chunks per group: chunk c is wave c % 16's, one lane each when assembled
+constexpr int kGroup = kChunks * kChunk;
+static_assert(kChunks == 64, "one lane per chunk");
 constexpr uint32_t kTop = 1u << 24;  // n at the end of a binade
 constexpr uint32_t kCap = 1u << 25;  // increments saturate here (64 of them still fit 32 bits)
 
@@ -279,13 +284,16 @@ typedef Terms Terms4 __attribute__((aligned(4)));  // rows start at any 4-byte b
 struct Inc {
   uint32_t d0, d1;
 };
-__device__ __forceinline__ Inc then(const Inc& a, const Inc& b) {
+__device__ __forceinline__ Inc then(Inc a, Inc b) {
   Inc c;
   c.d0 = min(a.d0 + ((a.d0 & 1u) ? b.d1 : b.d0), kCap);
   c.d1 = min(a.d1 + ((a.d1 & 1u) ? b.d0 : b.d1), kCap);
   return c;
 }
-__device__ __forceinline__ uint32_t advance(uint32_t n, const Inc& a) { return n + ((n & 1u) ? a.d1 : a.d0); }
+__device__ __forceinline__ uint32_t advance(uint32_t n, Inc a) {
+  const uint32_t d0 = a.d0, d1 = a.d1;
+  return n + ((n & 1u) ? d1 : d0);
+}
 
 // x of the lane that DPP control CTRL names, 0 (no increment) where it names none
 template <int CTRL, int ROWS = 0xF>
@@ -300,12 +308,41 @@ __device__ __forceinline__ void scan_step(Inc& x) {
 constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
 constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
 
-// Inclusive scan over each row of 16 lanes.
-__device__ __forceinline__ void scan_row(Inc& x) {
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float dpp_from_f(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xF, false));
+}
+
+// Inclusive scans over the wave.
+__device__ __forceinline__ float scan_sum(float x) {
+  x += dpp_from_f<kRowShr1>(x);
+  x += dpp_from_f<kRowShr2>(x);
+  x += dpp_from_f<kRowShr4>(x);
+  x += dpp_from_f<kRowShr8>(x);
+  x += dpp_from_f<kRowBcast15, 0xA>(x);
+  x += dpp_from_f<kRowBcast31, 0xC>(x);
+  return x;
+}
+__device__ __forceinline__ Inc scan_inc(Inc x) {
+  if (__builtin_amdgcn_ballot_w64(x.d0 != x.d1) == 0) {
+    // no tie in the wave: plain increments (64 * 2^25 at most)
+    uint32_t d = x.d0;
+    d += dpp_from<kRowShr1>(d);
+    d += dpp_from<kRowShr2>(d);
+    d += dpp_from<kRowShr4>(d);
+    d += dpp_from<kRowShr8>(d);
+    d += dpp_from<kRowBcast15, 0xA>(d);
+    d += dpp_from<kRowBcast31, 0xC>(d);
+    d = min(d, kCap);
+    return Inc{d, d};
+  }
   scan_step<kRowShr1>(x);
   scan_step<kRowShr2>(x);
   scan_step<kRowShr4>(x);
   scan_step<kRowShr8>(x);
+  scan_step<kRowBcast15, 0xA>(x);
+  scan_step<kRowBcast31, 0xC>(x);
+  return x;
 }
 
 // The ulp grid of a sum s >= 0: s = n * 2^exp.
@@ -328,55 +365,25 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
 
-// t / g, exact up to the cap (0 for a negative t, which is never taken from here)
-__device__ __forceinline__ float terms_on(float t, int exp) {
-  return __builtin_amdgcn_fmed3f(__builtin_amdgcn_ldexpf(t, -exp), 0.0f, static_cast<float>(kCap));
-}
-
-// Inclusive scan of the wave's terms on the grid 2^exp; lanes that are not
-// `active` contribute nothing.
-__device__ __forceinline__ Inc scan_terms(const Terms& t, bool active, int exp) {
-  uint32_t sum = 0;
-  bool tie = false;
+// Increments of n over a lane's terms, all >= 0, for a sum in the binade of
+// `base` >= 0: the terms added to base with its last bit cleared, and set.  A
+// sum that leaves the binade gives kCap.
+__device__ __forceinline__ Inc lane_inc(const Terms& t, float base) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, base);
+  float even = __builtin_bit_cast(float, u & ~1u), odd = __builtin_bit_cast(float, u | 1u);
 #pragma unroll
   for (int e = 0; e < kTerms; ++e) {
-    const float x = terms_on(t[e], exp);
-    const float q = __builtin_rintf(x);
-    tie |= fabsf(x - q) == 0.5f;
-    sum += static_cast<uint32_t>(q);
+    even += t[e];
+    odd += t[e];
   }
-  sum = active ? min(sum, kCap) : 0u;
-  if (__builtin_amdgcn_ballot_w64(tie && active) == 0) {
-    // no tie in the wave: plain increments (64 * 2^25 at most)
-    sum += dpp_from<kRowShr1>(sum);
-    sum += dpp_from<kRowShr2>(sum);
-    sum += dpp_from<kRowShr4>(sum);
-    sum += dpp_from<kRowShr8>(sum);
-    sum += dpp_from<kRowBcast15, 0xA>(sum);
-    sum += dpp_from<kRowBcast31, 0xC>(sum);
-    sum = min(sum, kCap);
-    return Inc{sum, sum};
-  }
-  Inc x = {0u, 0u};
-  if (active) {
-#pragma unroll
-    for (int e = 0; e < kTerms; ++e) {
-      const float v = terms_on(t[e], exp);
-      const float q = __builtin_rintf(v);
-      // a tie's even neighbour is q, its odd one the other
-      const uint32_t even = static_cast<uint32_t>(q);
-      const uint32_t odd = fabsf(v - q) == 0.5f ? 2u * static_cast<uint32_t>(v) + 1u - even : even;
-      x = then(x, Inc{even, odd});
-    }
-  }
-  scan_row(x);
-  scan_step<kRowBcast15, 0xA>(x);
-  scan_step<kRowBcast31, 0xC>(x);
-  return x;
+  const uint32_t a = __builtin_bit_cast(uint32_t, even), b = __builtin_bit_cast(uint32_t, odd);
+  // the last sum of base's binade is the first of the next; the lowest
+  // exponent has two binades of one grid
+  const uint32_t top = u < 0x00800000u ? 0x01000000u : (u & 0x7f800000u) + 0x00800000u;
+  return Inc{a <= top ? a - (u & ~1u) : kCap, b <= top ? b - (u | 1u) : kCap};
 }
 
-// Where a chain stands: the running sum and what it has found.  Uniform over
-// the workgroup.
+// Where a chain stands: the running sum and what it has found.
 struct Walk {
   float s;
   int tok;        // token found, valid with done
@@ -399,17 +406,43 @@ __device__ __forceinline__ bool is_hit(float s, float r) {
   return r < s;
 }
 
-// One wave takes its own 64 * kTerms terms (lane l: indices v0 .. v0 + kTerms)
-// from w to the end of them or to the token.
+// One wave takes a chunk of terms (lane l: indices v0 .. v0 + kTerms), `w` to
+// its end or to the token.  first: the row's first chunk, where the sum doubles
+// every few terms: the terms of its first kSerialLanes lanes are added in turn
+// from LDS (`first`).
+constexpr int kSerialLanes = 16;
 template <int MODE>
-__device__ void walk_wave(const Terms& t, int v0, int V, float r, bool bad, bool contrib, Walk& w) {
+__device__ __forceinline__ void walk_chunk(const Terms& t, int v0, int V, float r, float* first, Walk& w) {
   const int lane = threadIdx.x & 63;
-  for (int from = 0; from < 64;) {
+  bool bad = false, contrib = false;
+#pragma unroll
+  for (int e = 0; e < kTerms; ++e) {
+    bad |= !(t[e] >= 0.0f && t[e] < INFINITY);
+    contrib |= contributes<MODE>(t[e], v0 + e, V);
+  }
+  const uint64_t contribs = __builtin_amdgcn_ballot_w64(contrib);
+  const bool any_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+  int from = 0;
+  if (first != nullptr && !any_bad) {
+    if (lane < kSerialLanes) *reinterpret_cast<Terms*>(first + lane * kTerms) = t;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float x = w.s;
+#pragma unroll
+    for (int e = 0; e < kSerialLanes * kTerms; ++e) x += first[e];
+    if (!((contribs & ((1ull << kSerialLanes) - 1)) && is_hit<MODE>(x, r))) {  // (or the hit is found below)
+      w.s = lane_value(x, 0);
+      from = kSerialLanes;
+    }
+  }
+  while (from < 64) {
     int at = from;
     float s0 = w.s;
     if (on_grid(w.s)) {
       const Grid g = grid_of(w.s);
-      const Inc x = scan_terms(t, lane >= from, g.exp);
+      Inc x = {0u, 0u};
+      if (lane >= from && !bad) x = lane_inc(t, w.s);
+      x = scan_inc(x);
       const uint32_t n = advance(g.n, x);
       const float s = sum_of(n, g.exp);
       const bool stop = lane >= from && (n > kTop || bad || (contrib && is_hit<MODE>(s, r)));
@@ -447,9 +480,24 @@ __device__ void walk_wave(const Terms& t, int v0, int V, float r, bool bad, bool
   }
 }
 
+// What a wave says about a chunk.  The lanes up to the first doubtful one move
+// the sum on grid 2^exp by `head`; with at most kDoubtful doubtful lanes, `mid`
+// holds their terms (-0.0 beyond) and `tail` is the increment of the lanes
+// after them on grid 2^tail_exp.
+constexpr int kDoubtful = 2;
+enum Flags : int {
+  kParts = 1,    // has doubtful lanes
+  kWalkIt = 2,   // more of them, or a term that is negative or not finite
+  kHasHead = 4,  // lanes before the doubtful ones
+  kHasTail = 8,  // and after
+  kContrib = 16  // a contributing term
+};
 struct Shared {
-  uint32_t d0[2][kWaves], d1[2][kWaves];  // increments of each wave's terms, by pass parity
-  int flags[2][kWaves];                   // 1: has a contributing term, 2: has one off the grid
+  float total[kChunks];  // estimated sum of each chunk's terms
+  Inc head[kChunks], tail[kChunks];
+  int exp[kChunks], tail_exp[kChunks], flags[kChunks];
+  float mid[kChunks][kDoubtful * kTerms];
+  __attribute__((aligned(16))) float first[kSerialLanes * kTerms];
   Walk w;
 };
 
@@ -491,71 +539,155 @@ __device__ int chain(const float* __restrict__ a, const float* __restrict__ b, i
                      Shared& sh) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tid = threadIdx.x;
-  Walk w = {0.0f, 0, 0, 0};
   constexpr bool kDiff = MODE == kZ || MODE == kResidual;
-  Terms xa = load_terms(a, tid * kTerms, V);
-  Terms xb = kDiff ? load_terms(b, tid * kTerms, V) : Terms(0.0f);
-  int pass = 0;
-  for (int c0 = 0; c0 < V && !w.done; c0 += kTile) {
-    const int v0 = c0 + tid * kTerms;
-    const Terms t = make_terms<MODE>(xa, xb, Z, v0, V);
-    if (c0 + kTile < V) {  // the next tile's values travel while this one is summed
-      xa = load_terms(a, v0 + kTile, V);
-      if constexpr (kDiff) xb = load_terms(b, v0 + kTile, V);
-    }
-    bool bad = false, contrib = false;
+  auto terms_at = [&](int v0) {
+    const Terms xa = load_terms(a, v0, V);
+    const Terms xb = kDiff ? load_terms(b, v0, V) : Terms(0.0f);
+    return make_terms<MODE>(xa, xb, Z, v0, V);
+  };
+  Walk w = {0.0f, 0, 0, 0};
+  for (int c0 = 0; c0 < V && !w.done && w.s == w.s; c0 += kGroup) {
+    const int vw = c0 + (wave * 64 + lane) * kTerms;  // this lane's terms of its wave's first chunk
+    Terms xa[kTiles], xb[kTiles], t[kTiles];
 #pragma unroll
-    for (int e = 0; e < kTerms; ++e) {
-      bad |= !(t[e] >= 0.0f && t[e] < INFINITY);
-      contrib |= contributes<MODE>(t[e], v0 + e, V);
+    for (int j = 0; j < kTiles; ++j) {
+      xa[j] = load_terms(a, vw + j * kWaves * kChunk, V);
+      xb[j] = kDiff ? load_terms(b, vw + j * kWaves * kChunk, V) : Terms(0.0f);
     }
-    const int flags = (__builtin_amdgcn_ballot_w64(contrib) ? 1 : 0) | (__builtin_amdgcn_ballot_w64(bad) ? 2 : 0);
-    const int waves = min(kWaves, (V - c0 + 64 * kTerms - 1) / (64 * kTerms));  // waves with terms
-    int from = 0;         // first wave whose terms are still to be added
-    bool direct = c0 == 0;  // walk the next wave without a pass: the sum starts at 0 and doubles often
-    while (from < waves) {
-      int at = from;
-      if (!direct && on_grid(w.s)) {
-        const Grid g = grid_of(w.s);
-        const int buf = pass & 1;
-        ++pass;
-        Inc x = {0u, 0u};
-        if (wave >= from) x = scan_terms(t, true, g.exp);
-        if (lane == 63) {
-          sh.d0[buf][wave] = x.d0;
-          sh.d1[buf][wave] = x.d1;
-          sh.flags[buf][wave] = flags;
+    float upto[kTiles];  // estimated sum of the chunk up to this lane's end
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+      t[j] = make_terms<MODE>(xa[j], xb[j], Z, vw + j * kWaves * kChunk, V);
+      float mine = 0.0f;
+#pragma unroll
+      for (int e = 0; e < kTerms; ++e) mine += t[j][e];
+      upto[j] = scan_sum(mine);
+      if (lane == 63) sh.total[j * kWaves + wave] = upto[j];
+    }
+    __syncthreads();
+    const float chunk_end = w.s + scan_sum(sh.total[lane]);  // lane c: estimate at the end of chunk c
+    if (c0 == 0 && wave == 0) {
+      __builtin_amdgcn_s_setprio(3);  // everything waits for this walk
+      walk_chunk<MODE>(t[0], vw, V, r, sh.first, w);
+    }
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+      const int c = j * kWaves + wave;
+      if (c0 == 0 && c == 0) continue;  // walked
+      if (c0 + c * kChunk >= V) continue;
+      const float start = (c > 0 ? lane_value(chunk_end, max(c - 1, 0)) : w.s);
+      float mine = 0.0f, least = 0.0f;
+      bool contrib = false;
+#pragma unroll
+      for (int e = 0; e < kTerms; ++e) {
+        mine += t[j][e];
+        least = fminf(least, t[j][e]);
+        contrib |= contributes<MODE>(t[j][e], vw + j * kWaves * kChunk + e, V);
+      }
+      const bool bad = least < 0.0f || !(mine < INFINITY);  // (a NaN or infinite term shows in the sum)
+      // The estimate of where the sum stands before and after the lane's terms
+      // strays from the serial sum by far less than 2^-10; a wrong guess is
+      // noticed when the pieces are put together and costs a walk.
+      constexpr float kSlack = 1.0f / 1024.0f;
+      const float lo = start + (upto[j] - mine);
+      const int e0 = grid_of(lo * (1.0f - kSlack)).exp;
+      const int e1 = grid_of((start + upto[j]) * (1.0f + kSlack)).exp;
+      const uint64_t doubts = __builtin_amdgcn_ballot_w64(e0 != e1 || bad || !(lo >= 0.0f));
+      const int x0 = doubts ? __builtin_ctzll(doubts) : 64;  // doubtful lanes [x0, x1)
+      const int x1 = doubts ? 64 - __builtin_clzll(doubts) : 64;
+      const int head_exp = __builtin_amdgcn_readlane(e0, 0);
+      const int tail_exp = __builtin_amdgcn_readlane(e0, 63);
+      const bool in_doubt = lane >= x0 && lane < x1;
+      const Inc mine_inc = in_doubt ? Inc{0u, 0u} : lane_inc(t[j], lo);
+      Inc head = {lane < x0 ? mine_inc.d0 : 0u, lane < x0 ? mine_inc.d1 : 0u};
+      head = scan_inc(head);
+      int flags = (x0 > 0 ? kHasHead : 0) | (__builtin_amdgcn_ballot_w64(contrib) ? kContrib : 0);
+      // every lane of a run is on the run's grid
+      bool off = __builtin_amdgcn_ballot_w64((lane < x0 && e0 != head_exp) || (lane >= x1 && e0 != tail_exp)) != 0;
+      if (doubts) {
+        flags |= kParts;
+        off |= x1 - x0 > kDoubtful || __builtin_amdgcn_ballot_w64(bad) != 0;
+        if (x1 < 64) {
+          flags |= kHasTail;
+          Inc tail = {lane >= x1 ? mine_inc.d0 : 0u, lane >= x1 ? mine_inc.d1 : 0u};
+          tail = scan_inc(tail);
+          if (lane == 63) sh.tail[c] = tail;
         }
-        __syncthreads();
-        // lane l of each row of 16: wave l's end
-        Inc y = {sh.d0[buf][lane & 15], sh.d1[buf][lane & 15]};
-        const int f = sh.flags[buf][lane & 15];
-        scan_row(y);
-        const uint32_t n = advance(g.n, y);
-        const float s = sum_of(n, g.exp);
-        const bool stop = lane >= from && lane < waves &&
-                          (n > kTop || (f & 2) || ((f & 1) && is_hit<MODE>(s, r)));
-        const uint64_t stops = __builtin_amdgcn_ballot_w64(stop);
-        at = stops ? __builtin_ctzll(stops) : waves;
-        if (at > from) w.s = lane_value(s, at - 1);
-        if (at == waves) break;
-      } else if (!direct) {
-        __syncthreads();  // every wave has read sh.w
+        if (lane < kDoubtful * kTerms) sh.mid[c][lane] = -0.0f;
+        if (in_doubt && lane < x0 + kDoubtful) {
+#pragma unroll
+          for (int e = 0; e < kTerms; ++e) sh.mid[c][(lane - x0) * kTerms + e] = t[j][e];
+        }
       }
-      direct = false;
-      if (wave == at) {
-        walk_wave<MODE>(t, v0, V, r, bad, contrib, w);
-        if (lane == 0) sh.w = w;
+      if (off) flags |= kWalkIt;
+      if (lane == 63) sh.head[c] = head;  // (lanes from x0 on add nothing)
+      if (lane == 0) {
+        sh.exp[c] = head_exp;
+        sh.tail_exp[c] = tail_exp;
+        sh.flags[c] = flags;
       }
-      __syncthreads();
-      w = sh.w;
-      if (w.done || w.s != w.s) break;
-      from = at + 1;
     }
-    if (w.s != w.s) break;
+    __syncthreads();
+    // ---- wave 0 puts the pieces together: lane c has chunk c's ----
+    if (wave == 0) {
+      const int chunks = min(kChunks, (V - c0 + kChunk - 1) / kChunk);
+      int from = c0 == 0 ? 1 : 0;  // first chunk still to be added
+      const Inc my_head = sh.head[lane];
+      const int my_exp = sh.exp[lane], my_flags = sh.flags[lane];
+      while (from < chunks && !w.done && w.s == w.s) {
+        int at = from;
+        bool walk = !on_grid(w.s);
+        if (!walk) {
+          const Grid g = grid_of(w.s);
+          const bool mine = lane >= from && lane < chunks;
+          const Inc y = scan_inc(Inc{mine ? my_head.d0 : 0u, mine ? my_head.d1 : 0u});
+          const uint32_t n = advance(g.n, y);
+          const float s = sum_of(n, g.exp);
+          const bool stop = mine && ((my_flags & (kParts | kWalkIt)) || my_exp != g.exp || n > kTop ||
+                                     ((my_flags & kContrib) && is_hit<MODE>(s, r)));
+          const uint64_t stops = __builtin_amdgcn_ballot_w64(stop);
+          at = stops ? __builtin_ctzll(stops) : chunks;
+          if (at > from) w.s = lane_value(s, at - 1);
+          if (at == chunks) break;
+          const int fl = __builtin_amdgcn_readlane(my_flags, at);
+          walk = (fl & (kParts | kWalkIt)) != kParts;
+          if (!walk) {
+            // head, doubtful terms one by one, tail
+            const Inc head_at = sh.head[at], tail_at = sh.tail[at];
+            float x = w.s;
+            if (fl & kHasHead) {
+              const Grid h = grid_of(x);
+              const uint32_t m = advance(h.n, head_at);
+              walk = sh.exp[at] != h.exp || m > kTop;
+              x = sum_of(m, h.exp);
+            }
+#pragma unroll
+            for (int e = 0; e < kDoubtful * kTerms; ++e) x += sh.mid[at][e];
+            if (fl & kHasTail) {
+              const Grid q = grid_of(x);
+              const uint32_t m = advance(q.n, tail_at);
+              walk |= !on_grid(x) || sh.tail_exp[at] != q.exp || m > kTop;
+              x = sum_of(m, q.exp);
+            }
+            // sums only grow inside such a chunk: a hit anywhere shows at its end
+            walk |= !on_grid(x) || ((fl & kContrib) && is_hit<MODE>(x, r));
+            if (!walk) w.s = x;
+          }
+        }
+        if (walk) {
+          const int v0 = c0 + at * kChunk + lane * kTerms;
+          walk_chunk<MODE>(terms_at(v0), v0, V, r, nullptr, w);
+        }
+        from = at + 1;
+      }
+      if (lane == 0) sh.w = w;
+    }
+    __syncthreads();
+    w = sh.w;
+    __builtin_amdgcn_s_setprio(0);
+    // (sh.w and the records are written again only past the next group's first
+    // barrier, or, by the next chain, past its own)
   }
-  __syncthreads();  // every wave has read sh.w and the last pass before the next chain writes them
   if (sum) *sum = w.s;
   return w.done ? w.tok : 0;
 }
