@@ -253,14 +253,15 @@ __global__ __launch_bounds__(kThreads) void evict_kernel(const half_t* __restric
 // exact sum, and checks each piece against it: a wrong guess, a negative or
 // non-finite term or a hit sends that 512-term chunk to a walk, which locates
 // the lane concerned by the same scans and adds its terms in turn.  Only the
-// first chunk, where the sum doubles every few terms, is added serially.
+// row's first 128 terms, where the sum doubles every few, are all added in turn.
 //
-// Bound by the latency of these steps, about 7 us a row of 32000 (2 us its
-// first chunk, 2 us the assembly), not by bytes.  Two workgroups per row run
-// concurrently: Z, then the residual sample; the bonus token.  One lane adding
-// all the terms in turn from LDS, fed by a second wave, took 180 us for 16 rows
-// of 32000 words and K = 4; scans that restarted at each binade 63 us; this
-// takes FIG_AFTER us.
+// Bound by the latency of these steps, not by bytes: of about 15 us a row of
+// 32000 and scan, 4 us are the values' arrival, 2-3 us the first chunk, 3 us the
+// records and 7 us the assembly (0.8 us for each of its half-dozen crossings).
+// Two workgroups per row run concurrently: Z, then the residual sample; the
+// bonus token.  One lane adding all the terms in turn from LDS, fed by a second
+// wave, took 180 us for 16 rows of 32000 words and K = 4; scans that restarted
+// at each binade 63 us; this takes 33 us (128000 words: 77 us).
 namespace spec {
 
 constexpr int kMaxK = 8;      // SPEC_MAX_K (flash_attn_kernel.cu:3851)

@@ -233,10 +233,11 @@ def test_speculative_verify_non_monotone_rows(fa):
     _check_spec(fa, tp, dp, tok, rv, K)
 
 
-@pytest.mark.parametrize("V", [511, 512, 513, 8191, 8192, 8193, 16390, 40001])
+@pytest.mark.parametrize("V", [127, 128, 129, 511, 512, 513, 1025, 8193, 16390, 32767, 32768, 32769, 33281,
+                               70001])
 def test_speculative_verify_scan_edges(fa, V):
-    """The parallel scans of the serial sums at the edges of their waves (512
-    terms) and tiles (8192): exact (whole tokens) against the serial oracle,
+    """The parallel scans of the serial sums at the edges of their serial start
+    (128 terms), chunks (512) and groups (32768): exact (whole tokens) against the serial oracle,
     with a zero prefix, one term that lifts the sum by many binades, terms on
     ties, and r on a running sum of the bonus row."""
     B, K = 6, 1
