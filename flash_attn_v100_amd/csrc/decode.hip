@@ -52,8 +52,9 @@ constexpr unsigned kCounterSlotsDev = 65536;  // arrival counters in the workspa
 constexpr int kMaxChunk = 8192;                        // keys per split, upper bound
 constexpr int kChunkQuantum = FA_DEC_CHUNK_QUANTUM;    // split boundaries are multiples of this
 constexpr int kTargetBlocks = FA_DEC_TARGET_BLOCKS;    // aim for this many split workgroups
-// The paged kernel stages each split's page ids in LDS before its first load,
-// one extra memory round trip per split, so it prefers fewer, longer splits.
+// Statically planned paged calls (more sequences than the device plans) prefer
+// fewer, longer splits: each stages its page ids in LDS before its first load,
+// one extra memory round trip per split.
 #ifndef FA_DEC_PAGED_DIV
 #define FA_DEC_PAGED_DIV 4
 #endif
@@ -95,7 +96,12 @@ constexpr int kSplitMajorUnits = 64;  // fixed-length launches of at least this 
 #define FA_DEC_PREFETCH2 1
 #endif
 
-constexpr int kLptMaxSeqs = 512;      // longest-first ordering up to this many sequences
+// Continuous batching and paged calls plan their splits from the lengths on the
+// device up to this many sequences, and from this many statically planned
+// workgroups: a smaller grid is resident at once whatever its lengths, and the
+// planning costs it about 0.5 us (paged [4] to 4096 keys 12.7 -> 13.4).
+constexpr int kPlanMaxSeqs = 512;
+constexpr int kStaticMaxBlocks = 600;
 
 struct DecodeParams {
   const half_t* q;
@@ -119,12 +125,13 @@ struct DecodeParams {
   int fixed_len;               // decode / INT8: number of attended keys
   int chunk, num_splits, num_hg;
   int max_num_blocks, num_pages;
-  int lpt;                     // paged: serve sequences longest first
+  int ragged;                  // continuous batching, paged: plan from the lengths (ragged_item); 0: chunk, num_splits
   int absorb_tail;             // fixed-length: split 0 also takes the keys past S * chunk
   int seg1, seg_shift;         // contiguous modes: key v < seg1 is row v, later keys row v + seg_shift
                                // (seg_shift = 0: identity; sliding window: sink run, then window run)
   float scale_log2;            // (1/sqrt(D)) * log2(e)
   float scale;                 // 1/sqrt(D) (INT8 score formula)
+  int plan_len;                // ragged: longest plannable sequence (paged: the table row's tokens)
 };
 
 // Fetch the kernel arguments a mode uses at once: left to itself the compiler
@@ -146,10 +153,34 @@ __device__ __forceinline__ void preload_args(const DecodeParams& p) {
   }
   if constexpr (MODE == kModeInt8) asm volatile("" ::"s"(p.q_scale), "s"(p.k_scale), "s"(p.fixed_len), "s"(p.scale));
   if constexpr (MODE == kModeDecode) asm volatile("" ::"s"(p.fixed_len), "s"(p.seg1), "s"(p.seg_shift));
-  if constexpr (MODE == kModeCB) asm volatile("" ::"s"(p.lens), "s"(p.seg1), "s"(p.seg_shift));
+  if constexpr (MODE == kModeCB) asm volatile("" ::"s"(p.lens), "s"(p.seg1), "s"(p.seg_shift), "s"(p.ragged), "s"(p.plan_len));
   if constexpr (MODE == kModePaged)
-    asm volatile("" ::"s"(p.lens), "s"(p.lpt), "s"(p.block_table), "s"(p.bt_numel), "s"(p.max_num_blocks),
+    asm volatile("" ::"s"(p.lens), "s"(p.ragged), "s"(p.plan_len), "s"(p.block_table), "s"(p.bt_numel), "s"(p.max_num_blocks),
                  "s"(p.num_pages));
+}
+
+// Inclusive scans over a wave (gfx9 DPP row shifts and row broadcasts).
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp_shift(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_scan_add(int x) {
+  x += dpp_shift<0x111>(x);
+  x += dpp_shift<0x112>(x);
+  x += dpp_shift<0x114>(x);
+  x += dpp_shift<0x118>(x);
+  x += dpp_shift<0x142, 0xA>(x);
+  x += dpp_shift<0x143, 0xC>(x);
+  return x;
+}
+__device__ __forceinline__ int wave_scan_max(int x) {  // x >= 0
+  x = max(x, dpp_shift<0x111>(x));
+  x = max(x, dpp_shift<0x112>(x));
+  x = max(x, dpp_shift<0x114>(x));
+  x = max(x, dpp_shift<0x118>(x));
+  x = max(x, dpp_shift<0x142, 0xA>(x));
+  x = max(x, dpp_shift<0x143, 0xC>(x));
+  return x;
 }
 
 template <int MODE>
@@ -265,6 +296,122 @@ __device__ __forceinline__ int counter_index(int slot) {
   return (slot % kLines) * 32 + slot / kLines;
 }
 
+// A workgroup's share of a continuous-batching or paged call, planned from the
+// lengths (each wave for itself: no barrier, one read of the lengths, which
+// the static plan waits for as well).  A plan from the longest possible
+// sequence alone leaves half of its workgroups empty or short where lengths
+// are uniform, and each costs its slot a launch and a read of its length.
+// The chunk is the keys of all sequences over kRoundBlocks workgroups (one
+// resident round of two per CU); past kLongChunk keys, where one round leaves
+// the CUs unevenly loaded at its end, over kManyBlocks; and at least what the
+// workspace's S splits ask of the longest sequence.  Workgroups first take the
+// full chunks of all sequences, which are equal work, then the remainders.
+// Uniform lengths, D = 128, 32:8 heads (us, static -> planned): continuous
+// batching [64] to 8192 keys 185 -> 183, [128] to 4096 256 -> 191, [32] to 2048
+// 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 FIG_PAGED, [64] to
+// 8192 212 -> 189, [16] to 2048 26.1 -> 14.1, [64] to 1024 34 -> 26.7.  One round
+// against 2048 workgroups: paged [32] to 2048 28.9, 31.1; continuous batching
+// [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209, 183.
+constexpr int kRoundBlocks = 512;
+constexpr int kManyBlocks = 2048;
+template <int MODE>
+__host__ __device__ constexpr int long_chunk() { return MODE == kModePaged ? 768 : 1280; }
+
+struct RaggedItem {
+  int b;  // sequence (-1: none, the workgroup leaves)
+  int unit, split, splits, len, chunk;
+};
+
+// a / c for 0 <= a < 2^24 and c > 0 with inv = 1 / c
+__device__ __forceinline__ int div_by(int a, int c, float inv) {
+  int q = static_cast<int>(static_cast<float>(a) * inv);
+  const int r = a - q * c;
+  return q + (r >= c ? 1 : 0) - (r < 0 ? 1 : 0);
+}
+
+template <int MODE, int R>
+__device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) {
+  const int lane = threadIdx.x & 63;
+  const int per_seq = p.H_KV * p.num_hg;  // units per sequence
+  int len[R], plan[R], full[R], upto[R];
+  int sum = 0, mx = 0;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int q = lane + 64 * i;
+    len[i] = q < p.B ? seq_len_of<MODE>(p, q) : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    plan[i] = max(0, min(len[i], p.plan_len));
+    sum += plan[i];
+    mx = max(mx, plan[i]);
+  }
+  const int total = __builtin_amdgcn_readlane(wave_scan_add(sum), 63);
+  const int longest = __builtin_amdgcn_readlane(wave_scan_max(mx), 63);
+  const long long keys = static_cast<long long>(total) * per_seq;
+  const int round = static_cast<int>((keys + kRoundBlocks - 1) / kRoundBlocks);
+  const int many = static_cast<int>((keys + kManyBlocks - 1) / kManyBlocks);
+  const int want = max(min(round, max(long_chunk<MODE>(), many)), (longest + S - 1) / S);
+  RaggedItem it;
+  it.chunk = max(1, (want + kChunkQuantum - 1) / kChunkQuantum) * kChunkQuantum;
+  const float inv = 1.0f / static_cast<float>(it.chunk);
+  int all = 0;  // full chunks of every sequence
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    // (a sequence past its plannable length leaves at least one key to its
+    // last split, which takes the rest)
+    full[i] = div_by(len[i] > p.plan_len ? max(0, plan[i] - 1) : plan[i], it.chunk, inv);
+    upto[i] = all + wave_scan_add(full[i]);
+    all = __builtin_amdgcn_readlane(upto[i], 63);
+  }
+  const int item = static_cast<int>(blockIdx.x);
+  it.b = -1;
+  it.unit = it.split = it.splits = it.len = 0;
+  if (item < all * per_seq) {
+    const int c = item / per_seq;
+    it.unit = item % per_seq;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int before = upto[i] - full[i];
+      const uint64_t owner = __builtin_amdgcn_ballot_w64(c >= before && c < upto[i]);
+      if (owner != 0) {
+        const int l = __builtin_ctzll(owner);
+        it.b = l + 64 * i;
+        it.split = c - __builtin_amdgcn_readlane(before, l);
+        it.len = __builtin_amdgcn_readlane(len[i], l);
+        it.splits = __builtin_amdgcn_readlane(full[i] + (len[i] > full[i] * it.chunk ? 1 : 0), l);
+      }
+    }
+    return it;
+  }
+  // remainders: the sequences' in four classes of length, longest first, so
+  // that the short ones fill the end of the grid
+  int c = (item - all * per_seq) / per_seq;  // c-th remainder of that order
+  it.unit = (item - all * per_seq) % per_seq;
+#pragma unroll
+  for (int cls = 3; cls >= 0; --cls) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int rest = len[i] - full[i] * it.chunk;  // keys past the full chunks
+      const bool has = lane + 64 * i < p.B && (rest > 0 || len[i] <= 0);
+      const int quarter = rest * 4 > it.chunk * 3 ? 3 : (rest * 2 > it.chunk ? 2 : (rest * 4 > it.chunk ? 1 : 0));
+      const uint64_t in = __builtin_amdgcn_ballot_w64(has && quarter == cls);
+      const int count = __builtin_popcountll(in);
+      if (it.b < 0 && c < count) {
+        const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+            static_cast<uint32_t>(in >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(in), 0u)));
+        const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64((in >> lane & 1) && rank == c));
+        it.b = l + 64 * i;
+        it.split = __builtin_amdgcn_readlane(full[i], l);
+        it.len = __builtin_amdgcn_readlane(len[i], l);
+        it.splits = it.split + (it.len > 0 ? 1 : 0);
+      }
+      c -= it.b < 0 ? count : 0;
+    }
+  }
+  return it;
+}
+
 template <int DP, int GB, int MODE, int ROWS, bool LDSK>
 // Registers are the compiler's choice under the 256-thread bound (94-256
 // VGPRs across the instantiations, none spilling); asking for four waves per
@@ -294,42 +441,35 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
   constexpr bool kFixedLen = MODE == kModeDecode || MODE == kModeInt8 || MODE == kModeInt8KV;
   const int nslots = static_cast<int>(gridDim.x) / S;
   const bool split_major = kFixedLen && nslots >= kSplitMajorUnits;
-  const int split = split_major ? static_cast<int>(blockIdx.x) / nslots : blockIdx.x % S;
-  const int slot = split_major ? static_cast<int>(blockIdx.x) % nslots : blockIdx.x / S;  // this launch's counter slot
+  int split = split_major ? static_cast<int>(blockIdx.x) / nslots : blockIdx.x % S;
+  int slot = split_major ? static_cast<int>(blockIdx.x) % nslots : blockIdx.x / S;  // this launch's counter slot
+  const int D = p.D;
+  const int G = p.G;
+  const int tid = threadIdx.x;
+  int chunk = p.chunk;
+  int L, sb;  // keys of the sequence served; its splits that hold keys
+  bool to_end = false;  // this split takes every key up to L
+  constexpr bool kRagged = MODE == kModeCB || MODE == kModePaged;
+  if (kRagged && p.ragged) {
+    const RaggedItem it = p.B <= 64    ? ragged_item<MODE, 1>(p, S)
+                          : p.B <= 128 ? ragged_item<MODE, 2>(p, S)
+                                       : ragged_item<MODE, kPlanMaxSeqs / 64>(p, S);
+    if (it.b < 0) return;
+    chunk = it.chunk;
+    split = it.split;
+    L = it.len;
+    sb = it.splits;
+    to_end = split == sb - 1;
+    slot = it.b * p.H_KV * p.num_hg + it.unit;
+  }
   const int rest = p.unit_base + slot;  // (b, h_kv, head group) unit
   const int hg = rest % p.num_hg;
   const int pair = rest / p.num_hg;
   const int hkv = pair % p.H_KV;
-  const int D = p.D;
-  const int G = p.G;
+  const int b = pair / p.H_KV;  // sequence served
   const int g_base = hg * GB;
   const int g_valid = min(GB, G - g_base);  // heads of this group that exist
-
-  const int tid = threadIdx.x;
-  // Sequence served.  Paged decode with lpt set: unit rank r serves
-  // the sequence of rank r in descending length order (ties by index), so the
-  // longest sequences are dispatched first and the short ones fill the tail.
-  int b = pair / p.H_KV;
-  if constexpr (MODE == kModePaged) {
-    if (p.lpt) {
-      __shared__ int s_len[kLptMaxSeqs];
-      __shared__ int s_seq;
-      for (int i = tid; i < p.B; i += kDecThreads) s_len[i] = seq_len_of<MODE>(p, i);
-      __syncthreads();
-      const int r = b;
-      for (int i = tid; i < p.B; i += kDecThreads) {
-        const int li = s_len[i];
-        int rank = 0;
-        for (int j = 0; j < p.B; ++j) {
-          const int lj = s_len[j];
-          rank += (lj > li) || (lj == li && j < i);
-        }
-        if (rank == r) s_seq = i;
-      }
-      __syncthreads();
-      b = s_seq;
-    }
-  }
+  if (!(kRagged && p.ragged)) L = seq_len_of<MODE>(p, b);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // MFMA layout: lane = (key l16 of a 16-key tile, quarter q)
@@ -342,7 +482,6 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
   // accumulate are output columns past D, never stored.
   const int vcol = kChunks ? min(col, D - 8) : col;
 
-  const int L = seq_len_of<MODE>(p, b);
   // With absorb_tail (fixed-length calls only) the short remainder past
   // S * chunk (at most a quarter chunk) goes to split 0: [0, chunk + extra),
   // then split s takes [extra + s * chunk, +chunk).  Split 0 is dispatched
@@ -353,15 +492,15 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
   // Paged: the splits are planned over the table row (16 * max_num_blocks
   // tokens); a longer sequence keeps reading the flat table past its row, as
   // the reference does, and the last split takes all of those keys.
-  int k0 = split * p.chunk;
+  int k0 = split * chunk;
   int k1;
   if (FA_DEC_TAIL_FIRST && p.absorb_tail) {
-    const int extra = max(0, L - S * p.chunk);
-    k0 = split == 0 ? 0 : extra + split * p.chunk;
-    k1 = min(L, extra + (split + 1) * p.chunk);
+    const int extra = max(0, L - S * chunk);
+    k0 = split == 0 ? 0 : extra + split * chunk;
+    k1 = min(L, extra + (split + 1) * chunk);
   } else {
     const bool last_takes_rest = (p.absorb_tail || MODE == kModePaged) && split == S - 1;
-    k1 = last_takes_rest ? L : min(L, k0 + p.chunk);
+    k1 = to_end || last_takes_rest ? L : min(L, k0 + chunk);
   }
 
   if (k0 >= k1) {
@@ -380,7 +519,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
   }
 
   // Splits that hold keys of this sequence (>= 1 here, since k0 < k1).
-  const int sb = min(S, (L + p.chunk - 1) / p.chunk);
+  if (!(kRagged && p.ragged)) sb = min(S, (L + chunk - 1) / chunk);
 
   // Paged: the page ids of the keys [r0, r1) being walked are staged in LDS,
   // kMaxChunk keys per round (one round unless the sequence overruns its
@@ -1306,7 +1445,7 @@ static int check_common(const char* fn, int B, int H_Q, int H_KV, int D) {
 template <int MODE>
 static int target_blocks() {
   if constexpr (MODE == kModeInt8KV) return kTargetBlocksInt8KV;
-  return MODE == kModePaged ? kTargetBlocksPaged : (MODE == kModeCB ? kTargetBlocks : kTargetBlocksFixed);
+  return kTargetBlocksFixed;
 }
 // Split quantum of a fixed-length mode.
 template <int MODE>
@@ -1325,7 +1464,10 @@ constexpr long long kSmallGridBlocks = 256;
 template <int MODE>
 static DecodePlan plan_for(int B, int H_Q, int H_KV, int max_len, int D) {
   constexpr bool kFixed = MODE == kModeDecode || MODE == kModeInt8 || MODE == kModeInt8KV;
-  if (!kFixed) return make_plan(B, H_Q, H_KV, max_len, D, target_blocks<MODE>(), false, kChunkQuantum);
+  if (!kFixed) {
+    const int target = MODE == kModePaged && B > kPlanMaxSeqs ? kTargetBlocksPaged : kTargetBlocks;
+    return make_plan(B, H_Q, H_KV, max_len, D, target, false, kChunkQuantum);
+  }
   DecodePlan pl = make_plan(B, H_Q, H_KV, max_len, D, target_blocks<MODE>(), true, fixed_quantum<MODE>());
   const long long blocks = static_cast<long long>(B) * H_KV * pl.num_hg * pl.splits;
   if (blocks < kSmallGridBlocks) pl = make_plan(B, H_Q, H_KV, max_len, D, target_blocks<MODE>(), true, kSmallGridQuantum);
@@ -1347,13 +1489,7 @@ static int run_decode(const char* fn, DecodeParams p, int max_len, void* ws, siz
   if (pl.splits > kMaxSplits)
     return set_error(FA_ERR_UNSUPPORTED, "%s: %d keys per sequence exceed %d", fn, max_len, kMaxSplits * kMaxChunk);
   p.G = p.H_Q / p.H_KV;
-  // Longest first for paged decode only: its splits are long (a quarter of
-  // the continuous-batching target), so a long sequence dispatched late
-  // would trail the grid (config 4: 178 us with the order, 194 without).
-  // Continuous batching splits finely enough that no workgroup trails by
-  // much, and skipping the order's per-workgroup length ranking is faster
-  // there (config 3: 184.7 us without, 187.4 with).
-  p.lpt = MODE == kModePaged && p.B > 1 && p.B <= kLptMaxSeqs;
+  p.plan_len = max_len;
   p.chunk = pl.chunk;
   p.num_splits = pl.splits;
   p.num_hg = pl.num_hg;
@@ -1376,6 +1512,17 @@ static int run_decode(const char* fn, DecodeParams p, int max_len, void* ws, siz
   const int rows = !aligned || p.D % chunk != 0 ? kRowElems : (p.D == pl.dp ? kRowFull : kRowChunks);
   const long long units = static_cast<long long>(p.B) * p.H_KV * pl.num_hg;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!kFixed && units * pl.splits > kStaticMaxBlocks && p.B <= kPlanMaxSeqs &&
+      units <= static_cast<long long>(kCounterSlots)) {
+    // full chunks: at most kRoundBlocks, or kManyBlocks of at least
+    // long_chunk() keys each; then a remainder per unit
+    const long long full = std::max<long long>(
+        kRoundBlocks, std::min<long long>(kManyBlocks, units * max_len / long_chunk<MODE>()));
+    p.ragged = 1;
+    p.unit_base = 0;
+    dispatch<MODE>(pl, rows, p, static_cast<int>(full + units), st);
+    return check_launch(fn);
+  }
   for (long long u0 = 0; u0 < units; u0 += static_cast<long long>(kCounterSlots)) {
     const long long nu = units - u0 < static_cast<long long>(kCounterSlots) ? units - u0 : kCounterSlots;
     p.unit_base = static_cast<int>(u0);
