@@ -308,7 +308,7 @@ __device__ __forceinline__ int counter_index(int slot) {
 // full chunks of all sequences, which are equal work, then the remainders.
 // Uniform lengths, D = 128, 32:8 heads (us, static -> planned): continuous
 // batching [64] to 8192 keys 185 -> 183, [128] to 4096 256 -> 191, [32] to 2048
-// 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 FIG_PAGED, [64] to
+// 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 186 -> 185, [64] to
 // 8192 212 -> 189, [16] to 2048 26.1 -> 14.1, [64] to 1024 34 -> 26.7.  One round
 // against 2048 workgroups: paged [32] to 2048 28.9, 31.1; continuous batching
 // [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209, 183.

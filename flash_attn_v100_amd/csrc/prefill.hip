@@ -189,6 +189,15 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
   constexpr int CPR = DP / 8;                 // 16-byte chunks per row
   constexpr int IPW = TILE / 8 / 64 / kPreWaves;  // 16-byte copies per lane per tensor per tile
   constexpr float kRescaleLimit = 256.0f;  // 2^8: largest p before the max is refreshed
+  // Split blocks run one or two waves per SIMD with registers to spare: a tile's
+  // K fragments are all read before its first MFMA, and its V fragments before
+  // the softmax, so a read's latency is paid once and not per MFMA (the compiler
+  // otherwise waits for each read: causal [1,8,2048,128] 31.4 -> 27.9 us,
+  // [1,32:8,1024,128] 20.5 -> 19.0, [1,16,2048,256] 69.6 -> 62).  With three
+  // waves per SIMD the other waves cover it and the registers cost occupancy
+  // ([1,32:8,4096,128] 151 -> 168).
+  constexpr bool kEarlyReads = KS > 1;
+  static_assert(!kEarlyReads || (NBLK == 1 && RB == 1), "one 32 x 32 block of scores per wave");
   static_assert(IPW * 8 * 64 * kPreWaves == TILE, "tile must split evenly over the waves");
 
   __shared__ __attribute__((aligned(1024))) half_t smem[NS * 2 * Shape::TILE];
@@ -395,6 +404,16 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sacc[blk][rb][r] = 0.0f;
+    if constexpr (kEarlyReads) {
+      half8_t a[KK];
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) a[kk] = *lds_at<half8_t>(kaddr ^ (32 * kk));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+        sacc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk], qf[0][kk], sacc[0][0], 0, 0, 0);
+      return;
+    }
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
@@ -415,6 +434,25 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
   auto softmax_pv = [&](const int t, STile& sacc, const bool masked) {
     const int kt = t * kBK + kw;  // first key of the wave's keys in this tile
     const unsigned vaddr = lds_base + (t % NS) * kStageBytes + kTileBytes + v_lane + kw * DP * 2;
+    auto v_frag = [&](int db, int i) -> half8_t {
+      half4_t part[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const unsigned src = (vaddr ^ (16 * (4 * db ^ 2 * j))) + (16 * i + 8 * j) * DP * 2;
+        const short4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            const_cast<__attribute__((address_space(3))) short4_t*>(lds_at<short4_t>(src)));
+        part[j] = __builtin_bit_cast(half4_t, x);
+      }
+      return __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    half8_t vf[kEarlyReads ? DB : 1][2];
+    if constexpr (kEarlyReads) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) vf[db][i] = v_frag(db, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // ---- softmax (lane owns query row wq0 + 32 rb + l32) ----
     half8_t pf[RB][2 * NBLK];
 #pragma unroll
@@ -477,15 +515,7 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
     for (int db = 0; db < DB; ++db) {
 #pragma unroll
       for (int i = 0; i < 2 * NBLK; ++i) {
-        half4_t part[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const unsigned src = (vaddr ^ (16 * (4 * db ^ 2 * j))) + (16 * i + 8 * j) * DP * 2;
-          const short4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              const_cast<__attribute__((address_space(3))) short4_t*>(lds_at<short4_t>(src)));
-          part[j] = __builtin_bit_cast(half4_t, x);
-        }
-        const half8_t a = __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
+        const half8_t a = kEarlyReads ? vf[kEarlyReads ? db : 0][i & 1] : v_frag(db, i);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
 #ifdef FA_ABL_NOPV
