@@ -87,10 +87,10 @@ def test_prefill_chunk_rows_special_values(fa, d):
 
 @pytest.mark.parametrize("d", [64, 80, 128, 256])
 @pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("b,h,n", [(1, 32, 260), (3, 24, 129), (1, 70, 33), (2, 40, 321)])
+@pytest.mark.parametrize("b,h,n", [(1, 32, 260), (3, 24, 129), (1, 70, 33), (2, 40, 321), (1, 40, 1057)])
 def test_prefill_two_wave_blocks(fa, d, causal, b, h, n):
-    """Launches whose query blocks are shared by two waves (65 to 256 or, causal,
-    512 blocks of 128 rows) at the edges of their 64-row and 64-key tiles."""
+    """Launches whose query blocks are shared by two waves (65 to 256 blocks of 128
+    rows, or 512 of causal walks past 1024 keys) at the edges of their 64-row and 64-key tiles."""
     g = gen(d + n)
     q, k, v = (randn(g, b, h, n, d) for _ in range(3))
     out = fa.forward_fp16(*(t.to(DEV) for t in (q, k, v)), causal)
