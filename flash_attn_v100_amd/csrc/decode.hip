@@ -304,16 +304,21 @@ __device__ __forceinline__ int counter_index(int slot) {
 // The chunk is the keys of all sequences over kRoundBlocks workgroups (one
 // resident round of two per CU); past kLongChunk keys, where one round leaves
 // the CUs unevenly loaded at its end, over kManyBlocks; and at least what the
-// workspace's S splits ask of the longest sequence.  Workgroups first take the
-// full chunks of all sequences, which are equal work, then the remainders.
+// workspace's S splits ask of the longest sequence; paged calls of at least
+// kUnsplitUnits units, a resident round by themselves, run unsplit.  Workgroups
+// first take the full chunks of all sequences, which are equal work, then the
+// remainders, in classes of length, longest first.
 // Uniform lengths, D = 128, 32:8 heads (us, static -> planned): continuous
-// batching [64] to 8192 keys 185 -> 183, [128] to 4096 256 -> 191, [32] to 2048
-// 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 186 -> 185, [64] to
-// 8192 212 -> 189, [16] to 2048 26.1 -> 14.1, [64] to 1024 34 -> 26.7.  One round
-// against 2048 workgroups: paged [32] to 2048 28.9, 31.1; continuous batching
-// [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209, 183.
+// batching [64] to 8192 keys 171.7 -> 164.0, [128] to 4096 256 -> 191, [32] to 2048
+// 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 186.6 -> 184.8
+// (split in 2048 192), [64] to 8192 212 -> 189, [16] to 2048 26.1 -> 14.1, [64] to
+// 1024 34 -> 26.7.  One round against 2048 workgroups: paged [32] to 2048 28.9,
+// 31.1; continuous batching [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209,
+// 183.  Equal lengths pay for the remainders: continuous batching [16] to 2000-2048
+// 30.2 -> 32.4.
 constexpr int kRoundBlocks = 512;
 constexpr int kManyBlocks = 2048;
+constexpr int kUnsplitUnits = 768;  // a resident round of paged workgroups, three per CU
 template <int MODE>
 __host__ __device__ constexpr int long_chunk() { return MODE == kModePaged ? 768 : 1280; }
 
@@ -351,7 +356,10 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
   const long long keys = static_cast<long long>(total) * per_seq;
   const int round = static_cast<int>((keys + kRoundBlocks - 1) / kRoundBlocks);
   const int many = static_cast<int>((keys + kManyBlocks - 1) / kManyBlocks);
-  const int want = max(min(round, max(long_chunk<MODE>(), many)), (longest + S - 1) / S);
+  int want = max(min(round, max(long_chunk<MODE>(), many)), (longest + S - 1) / S);
+  // paged: enough sequences to fill the CUs run unsplit (no partials, no second
+  // staging of page ids), the length classes below keeping the tail short
+  if (MODE == kModePaged && p.B * per_seq >= kUnsplitUnits) want = longest;
   RaggedItem it;
   it.chunk = max(1, (want + kChunkQuantum - 1) / kChunkQuantum) * kChunkQuantum;
   const float inv = 1.0f / static_cast<float>(it.chunk);
@@ -384,18 +392,18 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
     }
     return it;
   }
-  // remainders: the sequences' in four classes of length, longest first, so
+  // remainders: the sequences' in eight classes of length, longest first, so
   // that the short ones fill the end of the grid
   int c = (item - all * per_seq) / per_seq;  // c-th remainder of that order
   it.unit = (item - all * per_seq) % per_seq;
 #pragma unroll
-  for (int cls = 3; cls >= 0; --cls) {
+  for (int cls = 7; cls >= 0; --cls) {
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int rest = len[i] - full[i] * it.chunk;  // keys past the full chunks
       const bool has = lane + 64 * i < p.B && (rest > 0 || len[i] <= 0);
-      const int quarter = rest * 4 > it.chunk * 3 ? 3 : (rest * 2 > it.chunk ? 2 : (rest * 4 > it.chunk ? 1 : 0));
-      const uint64_t in = __builtin_amdgcn_ballot_w64(has && quarter == cls);
+      const int eighth = max(0, min(7, static_cast<int>(static_cast<float>(rest) * (8.0f * inv))));
+      const uint64_t in = __builtin_amdgcn_ballot_w64(has && eighth == cls);
       const int count = __builtin_popcountll(in);
       if (it.b < 0 && c < count) {
         const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
