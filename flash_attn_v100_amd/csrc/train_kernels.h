@@ -531,6 +531,9 @@ __device__ __forceinline__ lds_ptr<float> part_slot(char* smem, int wave, int la
 // ---------------------------------------------------------------------------
 // Query-major kernel: MODE 0 = fp32 forward (O, optional LSE), MODE 1 = dQ + delta.
 // DC: columns computed (D <= DC <= DP).
+// Asking for two waves per SIMD at fp32 DP = 64 keeps the products in VGPRs and
+// the key-major kernel at two waves; without it they move to 32-64 AGPRs (with
+// the copies) and that kernel's 198 + 64 registers leave one wave per SIMD.
 template <typename T, int DP, int DC, int ROWS, int MODE, int SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && DP <= 64 ? 2 : 1))) void query_major_kernel(TrainParams p) {
   typedef typename Elem<T>::frag F;

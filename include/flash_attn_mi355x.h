@@ -90,8 +90,9 @@ size_t fa_backward_workspace_size(int B, int H, int N);
  * 1 <= D <= 128.  Two or three launches on `stream` (dQ with the row
  * statistic delta = rowsum(dout * out) into the workspace, then dK/dV, as one
  * pass or as a dV and a dK pass); deterministic (no atomics).  The workspace needs no initialisation.
- * Outside graph capture delta comes from a short kernel of its own and the
- * dK/dV work (fp16 at D > 64: the dV and the dK pass) runs on library-owned
+ * Large calls (fp16 at D > 64 past 512 blocks of 128 rows, fp32 at D > 64)
+ * outside graph capture take delta from a short kernel of its own and run the
+ * dK/dV work (fp16: the dV and the dK pass) on library-owned
  * side streams of the device (non-blocking, default priority) concurrently
  * with the dQ kernel, forked
  * from `stream` by events and joined back into it before return, so all of
@@ -267,9 +268,9 @@ int fa_token_eviction(const void* k, const void* v, const float* attn_scores,
  *   accepted draft tokens; at the first rejection i the residual sample
  *   (max(target - draft, 0) normalised, or target itself when that is all
  *   zero), the bonus token from target row i+1 and -1 after it; with no
- *   rejection the bonus from target row K.  Every running sum is accumulated
- *   serially in fp32 in vocabulary order, as the reference does; divisions are
- *   IEEE fp32.  Draft token ids outside [0, V) count as probability 0.
+ *   rejection the bonus from target row K.  Every running sum has the value of
+ *   a serial fp32 accumulation in vocabulary order, as in the reference;
+ *   divisions are IEEE fp32.  Draft token ids outside [0, V) count as probability 0.
  * Replaces speculative_verify_forward (flash_attn_kernel.cu:3972-4018), kernel
  * speculative_verify_kernel (:3853-3970).
  */
