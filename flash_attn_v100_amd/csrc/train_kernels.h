@@ -38,8 +38,8 @@
 //
 // The backward is dQ (each wave also computes delta_i = sum_d dO[i,d] O[i,d] of
 // its rows and publishes it in the workspace), then dK/dV, which reads delta;
-// large calls fork the passes onto side streams (backward_plan).  The key-major kernel does both
-// dK and dV in one pass when its registers allow (fp32, D <= 64 in fp16);
+// large calls fork the passes onto side streams (backward_plan).  The key-major
+// kernel does both dK and dV in one pass when its registers allow (fp32, D <= 64 in fp16);
 // otherwise (fp16, D > 64) one pass does dV (S and P only) and another dK
 // (S, dP, dS), so each fits 256 VGPRs and two waves share a SIMD.  No atomics:
 // every output element is written by exactly one lane, so results are
