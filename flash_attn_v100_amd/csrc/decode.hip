@@ -314,8 +314,11 @@ __device__ __forceinline__ int counter_index(int slot) {
 // (split in 2048 192), [64] to 8192 212 -> 189, [16] to 2048 26.1 -> 14.1, [64] to
 // 1024 34 -> 26.7.  One round against 2048 workgroups: paged [32] to 2048 28.9,
 // 31.1; continuous batching [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209,
-// 183.  Equal lengths pay for the remainders: continuous batching [16] to 2000-2048
-// 30.2 -> 32.4.
+// 183.  Equal lengths gain from the round size: continuous batching [16] of 2047
+// keys 28.8 -> 25.7, [64] of 4095 178 -> 167; paged [40,64:8] of 2999 pays 87.5 -> 90.9.
+// Past 128 sequences the planning itself is felt (R lengths a lane): four a lane
+// up to 256, and classes past the found one skipped, took uniform [256] to 1024
+// from 121.9 to 103.8 (paged 116.5 -> 101.3; static 125.5, 114.6).
 constexpr int kRoundBlocks = 512;
 constexpr int kManyBlocks = 2048;
 constexpr int kUnsplitUnits = 768;  // a resident round of paged workgroups, three per CU
@@ -398,6 +401,7 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
   it.unit = (item - all * per_seq) % per_seq;
 #pragma unroll
   for (int cls = 7; cls >= 0; --cls) {
+    if (it.b >= 0) break;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int rest = len[i] - full[i] * it.chunk;  // keys past the full chunks
@@ -461,6 +465,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
   if (kRagged && p.ragged) {
     const RaggedItem it = p.B <= 64    ? ragged_item<MODE, 1>(p, S)
                           : p.B <= 128 ? ragged_item<MODE, 2>(p, S)
+                          : p.B <= 256 ? ragged_item<MODE, 4>(p, S)
                                        : ragged_item<MODE, kPlanMaxSeqs / 64>(p, S);
     if (it.b < 0) return;
     chunk = it.chunk;
