@@ -1,6 +1,6 @@
 """Continuous batching and paged decode with the splits planned from the lengths
 on the device: every sequence against the CPU oracle, at batch sizes on both
-sides of the planner's register blocks (64, 128 and 512 sequences) and past it,
+sides of the planner's register blocks (64, 128, 256 and 512 sequences) and past it,
 with empty and negative lengths, lengths on and next to chunk boundaries, all
 equal, and one long sequence among short ones."""
 import pytest
@@ -33,7 +33,8 @@ def lengths(kind, b, n, g):
 @pytest.mark.parametrize("kind", ["uniform", "equal", "edges", "one_long"])
 @pytest.mark.parametrize("b,hq,hkv,n,d", [(64, 16, 4, 1100, 64), (65, 8, 4, 900, 128), (129, 8, 2, 1300, 64),
                                           (16, 32, 8, 2500, 64), (512, 2, 1, 600, 64), (513, 2, 1, 600, 64),
-                                          (3, 32, 8, 9000, 64)])
+                                          (3, 32, 8, 9000, 64), (256, 4, 2, 700, 64), (257, 4, 2, 700, 64),
+                                          (160, 8, 4, 256, 64)])  # the last: one split, not planned
 def test_continuous_batching_planned(fa, kind, b, hq, hkv, n, d):
     g = gen(b + n)
     q, k, v = randn(g, b, hq, 1, d), randn(g, b, hkv, n, d), randn(g, b, hkv, n, d)
@@ -49,7 +50,8 @@ def test_continuous_batching_planned(fa, kind, b, hq, hkv, n, d):
 
 @pytest.mark.parametrize("kind", ["uniform", "equal", "edges", "one_long", "overrun"])
 @pytest.mark.parametrize("b,hq,hkv,n,d", [(64, 16, 4, 1100, 64), (65, 8, 4, 900, 128), (129, 8, 2, 1300, 64),
-                                          (16, 32, 8, 2500, 64), (512, 2, 1, 600, 64), (513, 2, 1, 600, 64)])
+                                          (16, 32, 8, 2500, 64), (512, 2, 1, 600, 64), (513, 2, 1, 600, 64),
+                                          (256, 4, 2, 700, 64), (257, 4, 2, 700, 64)])
 def test_paged_planned(fa, kind, b, hq, hkv, n, d):
     g = gen(b + n + 1)
     blocks = (n + 15) // 16
