@@ -396,7 +396,7 @@ struct Walk {
 // past V) is -0.0, which leaves the sum unchanged and is never a hit; one that
 // does has its sign bit clear.  Past V every mode has -0.0.
 template <int MODE>
-__device__ __forceinline__ bool contributes(float t, int v, int V) {
+__device__ __forceinline__ bool contributes(float t, uint32_t v, uint32_t V) {
   if constexpr (MODE == kResidual) return !__builtin_signbit(t);
   return v < V;
 }
@@ -413,7 +413,7 @@ __device__ __forceinline__ bool is_hit(float s, float r) {
 // from LDS (`first`).
 constexpr int kSerialLanes = 16;
 template <int MODE>
-__device__ __forceinline__ void walk_chunk(const Terms& t, int v0, int V, float r, float* first, Walk& w) {
+__device__ __forceinline__ void walk_chunk(const Terms& t, uint32_t v0, uint32_t V, float r, float* first, Walk& w) {
   const int lane = threadIdx.x & 63;
   bool bad = false, contrib = false;
 #pragma unroll
@@ -463,10 +463,10 @@ __device__ __forceinline__ void walk_chunk(const Terms& t, int v0, int V, float 
 #pragma unroll
     for (int e = 0; e < kTerms; ++e) {
       s += t[e];
-      const int v = v0 + e;
+      const uint32_t v = v0 + e;
       if (tok < 0 && contributes<MODE>(t[e], v, V) && is_hit<MODE>(s, r)) {
         if (v == 0) zero_hit = 1;
-        else tok = v;
+        else tok = static_cast<int>(v);
       }
     }
     w.s = lane_value(s, at);
@@ -503,7 +503,7 @@ struct Shared {
 };
 
 // row[v0 .. v0 + kTerms), 0 past V
-__device__ __forceinline__ Terms load_terms(const float* row, int v0, int V) {
+__device__ __forceinline__ Terms load_terms(const float* row, uint32_t v0, uint32_t V) {
   Terms x;
   if (v0 + kTerms <= V) return *reinterpret_cast<const Terms4*>(row + v0);
 #pragma unroll
@@ -513,7 +513,7 @@ __device__ __forceinline__ Terms load_terms(const float* row, int v0, int V) {
 
 // The chain's terms from row values a (and b).
 template <int MODE>
-__device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, float Z, int v0, int V) {
+__device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, float Z, uint32_t v0, uint32_t V) {
   Terms t;
 #pragma unroll
   for (int e = 0; e < kTerms; ++e) {
@@ -534,21 +534,22 @@ __device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, floa
 //  kBonus:    cs += a; hit when cs >= r.
 // Returns the reference's token: the first hit, or the next hit if the first
 // is index 0 (0 without hits).  Every wave takes the same path through the
-// barriers: what decides it is read from LDS after one.
+// barriers: what decides it is read from LDS after one.  Indices are unsigned:
+// the last group's ends pass 2^31 when V is within a group of it.
 template <int MODE>
-__device__ int chain(const float* __restrict__ a, const float* __restrict__ b, int V, float Z, float r, float* sum,
+__device__ int chain(const float* __restrict__ a, const float* __restrict__ b, uint32_t V, float Z, float r, float* sum,
                      Shared& sh) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr bool kDiff = MODE == kZ || MODE == kResidual;
-  auto terms_at = [&](int v0) {
+  auto terms_at = [&](uint32_t v0) {
     const Terms xa = load_terms(a, v0, V);
     const Terms xb = kDiff ? load_terms(b, v0, V) : Terms(0.0f);
     return make_terms<MODE>(xa, xb, Z, v0, V);
   };
   Walk w = {0.0f, 0, 0, 0};
-  for (int c0 = 0; c0 < V && !w.done && w.s == w.s; c0 += kGroup) {
-    const int vw = c0 + (wave * 64 + lane) * kTerms;  // this lane's terms of its wave's first chunk
+  for (uint32_t c0 = 0; c0 < V && !w.done && w.s == w.s; c0 += kGroup) {
+    const uint32_t vw = c0 + (wave * 64 + lane) * kTerms;  // this lane's terms of its wave's first chunk
     Terms xa[kTiles], xb[kTiles], t[kTiles];
 #pragma unroll
     for (int j = 0; j < kTiles; ++j) {
@@ -631,7 +632,7 @@ __device__ int chain(const float* __restrict__ a, const float* __restrict__ b, i
     __syncthreads();
     // ---- wave 0 puts the pieces together: lane c has chunk c's ----
     if (wave == 0) {
-      const int chunks = min(kChunks, (V - c0 + kChunk - 1) / kChunk);
+      const int chunks = static_cast<int>(min(static_cast<uint32_t>(kChunks), (V - c0 + kChunk - 1) / kChunk));
       int from = c0 == 0 ? 1 : 0;  // first chunk still to be added
       const Inc my_head = sh.head[lane];
       const int my_exp = sh.exp[lane], my_flags = sh.flags[lane];
@@ -676,7 +677,7 @@ __device__ int chain(const float* __restrict__ a, const float* __restrict__ b, i
           }
         }
         if (walk) {
-          const int v0 = c0 + at * kChunk + lane * kTerms;
+          const uint32_t v0 = c0 + at * kChunk + lane * kTerms;
           walk_chunk<MODE>(terms_at(v0), v0, V, r, nullptr, w);
         }
         from = at + 1;

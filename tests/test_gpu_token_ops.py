@@ -258,6 +258,22 @@ def test_speculative_verify_scan_edges(fa, V):
     _check_spec(fa, tp, dp, tok, rv, K)
 
 
+def test_speculative_verify_vocabulary_near_the_int32_limit(fa):
+    """A row whose last scan group reaches past index 2^31: every scan stops at the
+    row's end.  The tokens follow from the few non-zero terms; r = 2 is reached
+    by no sum, so that scan runs the whole row and finds nothing."""
+    V = 2 ** 31 - 4096
+    if torch.cuda.mem_get_info()[0] < 40e9:
+        pytest.skip("needs 26 GB for the rows")
+    tp, dp = torch.zeros(1, 2, V, device="cuda"), torch.zeros(1, 1, V, device="cuda")
+    tp[0, 0, V - 5] = 1.0
+    tp[0, 1, 100], tp[0, 1, V - 2] = 0.25, 0.75
+    tok = torch.tensor([[3]], device="cuda")
+    for r, want in ((0.5, [V - 5, V - 2]), (2.0, [0, 0])):
+        acc, out = fa.speculative_verify(tp, dp, tok, torch.tensor([[r]], device="cuda"), 1)
+        assert acc.tolist() == [0] and out[0].tolist() == want
+
+
 def test_speculative_verify_validation(fa):
     tp = torch.rand(1, 3, 10, device="cuda")
     dp = torch.rand(1, 2, 10, device="cuda")
