@@ -388,7 +388,6 @@ __device__ __forceinline__ Inc lane_inc(const Terms& t, float base) {
 struct Walk {
   float s;
   int tok;        // token found, valid with done
-  int zero_hit;   // a hit at index 0 was seen, the next hit decides
   int done;
 };
 
@@ -459,18 +458,14 @@ __device__ __forceinline__ void walk_chunk(const Terms& t, uint32_t v0, uint32_t
     }
     // lane `at` adds its terms one by one (every lane does, its own are kept)
     float s = s0;
-    int tok = -1, zero_hit = w.zero_hit;
+    int tok = -1;
 #pragma unroll
     for (int e = 0; e < kTerms; ++e) {
       s += t[e];
       const uint32_t v = v0 + e;
-      if (tok < 0 && contributes<MODE>(t[e], v, V) && is_hit<MODE>(s, r)) {
-        if (v == 0) zero_hit = 1;
-        else tok = static_cast<int>(v);
-      }
+      if (tok < 0 && v > 0 && contributes<MODE>(t[e], v, V) && is_hit<MODE>(s, r)) tok = static_cast<int>(v);
     }
     w.s = lane_value(s, at);
-    w.zero_hit = __builtin_amdgcn_readlane(zero_hit, at);
     tok = __builtin_amdgcn_readlane(tok, at);
     if (tok >= 0) {
       w.tok = tok;
@@ -532,8 +527,8 @@ __device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, floa
 //  kResidual: cs += (a - b) / Z where a - b > 0; hit at such v when r < cs.
 //  kPrefix:   cs += a; hit when r < cs.
 //  kBonus:    cs += a; hit when cs >= r.
-// Returns the reference's token: the first hit, or the next hit if the first
-// is index 0 (0 without hits).  Every wave takes the same path through the
+// Returns the reference's token: the first hit past index 0 (there, a hit at
+// index 0 is replaced by the next one), 0 without one.  Every wave takes the same path through the
 // barriers: what decides it is read from LDS after one.  Indices are unsigned:
 // the last group's ends pass 2^31 when V is within a group of it.
 template <int MODE>
@@ -547,7 +542,7 @@ __device__ int chain(const float* __restrict__ a, const float* __restrict__ b, u
     const Terms xb = kDiff ? load_terms(b, v0, V) : Terms(0.0f);
     return make_terms<MODE>(xa, xb, Z, v0, V);
   };
-  Walk w = {0.0f, 0, 0, 0};
+  Walk w = {0.0f, 0, 0};
   for (uint32_t c0 = 0; c0 < V && !w.done && w.s == w.s; c0 += kGroup) {
     const uint32_t vw = c0 + (wave * 64 + lane) * kTerms;  // this lane's terms of its wave's first chunk
     Terms xa[kTiles], xb[kTiles], t[kTiles];
