@@ -261,7 +261,10 @@ __global__ __launch_bounds__(kThreads) void evict_kernel(const half_t* __restric
 // Two workgroups per row run concurrently: Z, then the residual sample; the
 // bonus token.  One lane adding all the terms in turn from LDS, fed by a second
 // wave, took 180 us for 16 rows of 32000 words and K = 4; scans that restarted
-// at each binade 63 us; this takes 33 us (128000 words: 77 us).
+// at each binade 63 us; this takes 31-35 us (128000 words: 77-80 us).  The scans
+// are compiled into the kernel: as calls, which reach LDS by generic addresses
+// and keep registers in scratch, all-accepted batches (the bonus scan alone) took
+// 19.2 us against 15.8.
 namespace spec {
 
 constexpr int kMaxK = 8;      // SPEC_MAX_K (flash_attn_kernel.cu:3851)
@@ -532,7 +535,7 @@ __device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, floa
 // barriers: what decides it is read from LDS after one.  Indices are unsigned:
 // the last group's ends pass 2^31 when V is within a group of it.
 template <int MODE>
-__device__ int chain(const float* __restrict__ a, const float* __restrict__ b, uint32_t V, float Z, float r, float* sum,
+__device__ __forceinline__ int chain(const float* __restrict__ a, const float* __restrict__ b, uint32_t V, float Z, float r, float* sum,
                      Shared& sh) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
