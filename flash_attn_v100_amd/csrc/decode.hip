@@ -302,7 +302,7 @@ __device__ __forceinline__ int counter_index(int slot) {
 // sequence alone leaves half of its workgroups empty or short where lengths
 // are uniform, and each costs its slot a launch and a read of its length.
 // The chunk is the keys of all sequences over kRoundBlocks workgroups (one
-// resident round of two per CU); past kLongChunk keys, where one round leaves
+// resident round of two per CU); past long_chunk() keys, where one round leaves
 // the CUs unevenly loaded at its end, over kManyBlocks; and at least what the
 // workspace's S splits ask of the longest sequence; paged calls of at least
 // kUnsplitUnits units, a resident round by themselves, run unsplit.  Workgroups
@@ -316,9 +316,15 @@ __device__ __forceinline__ int counter_index(int slot) {
 // 31.1; continuous batching [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209,
 // 183.  Equal lengths gain from the round size: continuous batching [16] of 2047
 // keys 28.8 -> 25.7, [64] of 4095 178 -> 167; paged [40,64:8] of 2999 pays 87.5 -> 90.9.
-// Past 128 sequences the planning itself is felt (R lengths a lane): four a lane
-// up to 256, and classes past the found one skipped, took uniform [256] to 1024
-// from 121.9 to 103.8 (paged 116.5 -> 101.3; static 125.5, 114.6).
+// The planning itself is felt where sequences are short or many (R lengths a
+// lane), so the class of the remainder sought is found from counts that one
+// scan adds up over the wave, and only its members are looked through; with
+// every class counted by a ballot a length, in code unrolled 8 R times, one
+// long sequence among short ones lost to the static plan (static, ballots,
+// scan): continuous batching [400,32:4] to 1500 33.6, 53.1, 32.4, [200] to 1500
+// 27.7, 34.7, 24.9, [128] to 2000 35.4, 19.1, 16.3; uniform [256] to 1024 122.1,
+// 100.8, 93.0, paged [256] to 2048 183.0, 173.8, 170.8.  Left: sequences of a few
+// keys beside one of 600, [400,32:4], 22.2, 40.9, 27.1.
 constexpr int kRoundBlocks = 512;
 constexpr int kManyBlocks = 2048;
 constexpr int kUnsplitUnits = 768;  // a resident round of paged workgroups, three per CU
@@ -378,6 +384,9 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
   const int item = static_cast<int>(blockIdx.x);
   it.b = -1;
   it.unit = it.split = it.splits = it.len = 0;
+  uint64_t in = 0;      // the lanes that may hold the item's sequence, in block `base` / 64,
+  int base = 0;         // and these lanes' values there
+  int its_len = 0, its_full = 0, its_before = 0;
   if (item < all * per_seq) {
     const int c = item / per_seq;
     it.unit = item % per_seq;
@@ -386,41 +395,73 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
       const int before = upto[i] - full[i];
       const uint64_t owner = __builtin_amdgcn_ballot_w64(c >= before && c < upto[i]);
       if (owner != 0) {
-        const int l = __builtin_ctzll(owner);
-        it.b = l + 64 * i;
-        it.split = c - __builtin_amdgcn_readlane(before, l);
-        it.len = __builtin_amdgcn_readlane(len[i], l);
-        it.splits = __builtin_amdgcn_readlane(full[i] + (len[i] > full[i] * it.chunk ? 1 : 0), l);
+        in = owner;
+        base = 64 * i;
+        its_len = len[i];
+        its_full = full[i];
+        its_before = before;
       }
     }
+    const int l = __builtin_ctzll(in);
+    it.b = base + l;
+    it.split = c - __builtin_amdgcn_readlane(its_before, l);
+    it.len = __builtin_amdgcn_readlane(its_len, l);
+    it.splits = __builtin_amdgcn_readlane(its_full, l);
+    it.splits += it.len > it.splits * it.chunk ? 1 : 0;
     return it;
   }
   // remainders: the sequences' in eight classes of length, longest first, so
   // that the short ones fill the end of the grid
   int c = (item - all * per_seq) / per_seq;  // c-th remainder of that order
   it.unit = (item - all * per_seq) % per_seq;
+  int cls[R];            // class of the lane's sequences (-1: no remainder)
+  uint64_t mine = 0;     // how many it has of each: 8 bits a class
 #pragma unroll
-  for (int cls = 7; cls >= 0; --cls) {
-    if (it.b >= 0) break;
+  for (int i = 0; i < R; ++i) {
+    const int rest = len[i] - full[i] * it.chunk;  // keys past the full chunks
+    const bool has = lane + 64 * i < p.B && (rest > 0 || len[i] <= 0);
+    const int eighth = max(0, min(7, static_cast<int>(static_cast<float>(rest) * (8.0f * inv))));
+    cls[i] = has ? eighth : -1;
+    mine += has ? 1ull << (8 * eighth) : 0ull;
+  }
+  // the wave's: 16 bits a class, classes 0 2 | 1 3 | 4 6 | 5 7
+  uint32_t counts[4];
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const int rest = len[i] - full[i] * it.chunk;  // keys past the full chunks
-      const bool has = lane + 64 * i < p.B && (rest > 0 || len[i] <= 0);
-      const int eighth = max(0, min(7, static_cast<int>(static_cast<float>(rest) * (8.0f * inv))));
-      const uint64_t in = __builtin_amdgcn_ballot_w64(has && eighth == cls);
-      const int count = __builtin_popcountll(in);
-      if (it.b < 0 && c < count) {
-        const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-            static_cast<uint32_t>(in >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(in), 0u)));
-        const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64((in >> lane & 1) && rank == c));
-        it.b = l + 64 * i;
-        it.split = __builtin_amdgcn_readlane(full[i], l);
-        it.len = __builtin_amdgcn_readlane(len[i], l);
-        it.splits = it.split + (it.len > 0 ? 1 : 0);
-      }
-      c -= it.b < 0 ? count : 0;
+  for (int j = 0; j < 4; ++j)
+    counts[j] = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+        wave_scan_add(static_cast<int>(static_cast<uint32_t>(mine >> (8 * (j & 1) + 32 * (j >> 1))) & 0x00ff00ffu)), 63));
+  int its_cls = -1;
+#pragma unroll
+  for (int k = 7; k >= 0; --k) {
+    const int count = static_cast<int>(counts[2 * (k >> 2) + (k & 1)] >> (16 * (k >> 1 & 1)) & 0xffffu);
+    if (its_cls < 0) {
+      if (c < count) its_cls = k;
+      else c -= count;
     }
   }
+  if (its_cls < 0) return it;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const uint64_t of_cls = __builtin_amdgcn_ballot_w64(cls[i] == its_cls);
+    const int count = __builtin_popcountll(of_cls);
+    if (in == 0) {
+      if (c < count) {
+        in = of_cls;
+        base = 64 * i;
+        its_len = len[i];
+        its_full = full[i];
+      } else {
+        c -= count;
+      }
+    }
+  }
+  const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+      static_cast<uint32_t>(in >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(in), 0u)));
+  const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64((in >> lane & 1) && rank == c));
+  it.b = base + l;
+  it.len = __builtin_amdgcn_readlane(its_len, l);
+  it.split = __builtin_amdgcn_readlane(its_full, l);
+  it.splits = it.split + (it.len > 0 ? 1 : 0);
   return it;
 }
 

@@ -55,10 +55,10 @@ def test_continuous_batching_planned(fa, kind, b, hq, hkv, n, d):
 def test_paged_planned(fa, kind, b, hq, hkv, n, d):
     g = gen(b + n + 1)
     blocks = (n + 15) // 16
-    pages = b * blocks
+    pages = min(b * blocks, 8192)  # (long tables share pages)
     q = randn(g, b, hq, 1, d)
     k, v = randn(g, pages, hkv, 16, d), randn(g, pages, hkv, 16, d)
-    table = torch.randperm(pages, generator=g).to(torch.int32).view(b, blocks)
+    table = torch.randperm(b * blocks, generator=g).remainder(pages).to(torch.int32).view(b, blocks)
     lens = (lengths("uniform" if kind == "overrun" else kind, b, n, g) + 1).to(torch.int32)
     lens[0] = 0
     if kind == "overrun":  # reads on into the next table row, as the flat table does
@@ -76,6 +76,38 @@ def test_paged_planned(fa, kind, b, hq, hkv, n, d):
         assert_close(out[i:i + 1], A.decode(q[i:i + 1], ks, vs, True, ln - 1), what=f"{kind} sequence {i}, {ln}")
     again = fa.forward_paged_decode_gqa_fp16(*(t.to(DEV) for t in (q, k, v, table, lens)), blocks)
     assert torch.equal(torch.nan_to_num(out), torch.nan_to_num(again))
+
+
+@pytest.mark.parametrize("kind", ["uniform", "equal", "edges", "one_long"])
+@pytest.mark.parametrize("b,hq,hkv,n,d", [(128, 8, 8, 700, 64), (256, 8, 4, 500, 64)])
+def test_paged_planned_equals_single_sequences(fa, kind, b, hq, hkv, n, d):
+    """Every sequence of a batch that fills the CUs against a call with that
+    sequence alone, whose splits come from its table."""
+    g = gen(b + n + 2)
+    blocks = (n + 15) // 16
+    pages = min(b * blocks, 8192)
+    q, k, v = (t.to(DEV) for t in (randn(g, b, hq, 1, d), randn(g, pages, hkv, 16, d), randn(g, pages, hkv, 16, d)))
+    table = torch.randint(0, pages, (b, blocks), generator=g).to(torch.int32).to(DEV)
+    lens = (lengths(kind, b, n, g) + 1).to(torch.int32).to(DEV)
+    lens[1] = 0
+    out = fa.forward_paged_decode_gqa_fp16(q, k, v, table, lens, blocks)
+    one = [fa.forward_paged_decode_gqa_fp16(q[i:i + 1], k, v, table[i:i + 1], lens[i:i + 1], blocks) for i in range(b)]
+    assert_close(out, torch.cat(one), what=f"{kind} [{b}] to {n}")
+
+
+@pytest.mark.parametrize("kind", ["uniform", "equal", "edges", "one_long"])
+@pytest.mark.parametrize("b,hq,hkv,n,d", [(40, 16, 4, 1100, 64), (128, 8, 4, 900, 64), (200, 8, 4, 900, 64),
+                                          (400, 8, 4, 600, 64)])
+def test_continuous_batching_planned_equals_single_sequences(fa, kind, b, hq, hkv, n, d):
+    """Every sequence of a planned batch against a call with that sequence alone."""
+    g = gen(b + n + 3)
+    q, k, v = (t.to(DEV) for t in (randn(g, b, hq, 1, d), randn(g, b, hkv, n, d), randn(g, b, hkv, n, d)))
+    lens = lengths(kind, b, n, g).to(torch.int32).to(DEV)
+    lens[1] = -1
+    out = fa.forward_continuous_batching_fp16(q, k, v, lens, True)
+    one = [fa.forward_continuous_batching_fp16(q[i:i + 1], k[i:i + 1], v[i:i + 1], lens[i:i + 1], True)
+           for i in range(b)]
+    assert_close(out, torch.cat(one), what=f"{kind} [{b}] to {n}")
 
 
 def test_planned_calls_replay_with_other_lengths(fa):
