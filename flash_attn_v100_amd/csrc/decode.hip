@@ -305,9 +305,10 @@ __device__ __forceinline__ int counter_index(int slot) {
 // resident round of two per CU); past long_chunk() keys, where one round leaves
 // the CUs unevenly loaded at its end, over kManyBlocks; and at least what the
 // workspace's S splits ask of the longest sequence; paged calls of at least
-// kUnsplitUnits units, a resident round by themselves, run unsplit.  Workgroups
-// first take the full chunks of all sequences, which are equal work, then the
-// remainders, in classes of length, longest first.
+// kUnsplitUnits units, a resident round by themselves, run unsplit where no
+// sequence is long against the batch.  Workgroups first take the full chunks of
+// all sequences, which are equal work, then the remainders, in classes of
+// length, longest first.
 // Uniform lengths, D = 128, 32:8 heads (us, static -> planned): continuous
 // batching [64] to 8192 keys 171.7 -> 164.0, [128] to 4096 256 -> 191, [32] to 2048
 // 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 186.6 -> 184.8
@@ -328,6 +329,7 @@ __device__ __forceinline__ int counter_index(int slot) {
 constexpr int kRoundBlocks = 512;
 constexpr int kManyBlocks = 2048;
 constexpr int kUnsplitUnits = 768;  // a resident round of paged workgroups, three per CU
+constexpr int kSplitCost = 256;     // keys that a workgroup walks in the time that splitting costs it
 template <int MODE>
 __host__ __device__ constexpr int long_chunk() { return MODE == kModePaged ? 768 : 1280; }
 
@@ -367,8 +369,17 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
   const int many = static_cast<int>((keys + kManyBlocks - 1) / kManyBlocks);
   int want = max(min(round, max(long_chunk<MODE>(), many)), (longest + S - 1) / S);
   // paged: enough sequences to fill the CUs run unsplit (no partials, no second
-  // staging of page ids), the length classes below keeping the tail short
-  if (MODE == kModePaged && p.B * per_seq >= kUnsplitUnits) want = longest;
+  // staging of page ids), the length classes below keeping the tail short, if
+  // the longest walk ends within the call: a workgroup alone walks 64 keys a us
+  // and a full chip takes 12400 keys a us, so a walk is as long as the call at
+  // 2.6 shares of a round; beyond two, and what a split costs, it would trail
+  // it.  (us, split at kMaxChunk, all unsplit, this rule; 32:8 heads, D = 128)
+  // [128] one of 4096 keys, mean 66: 67.7, 64.5, 22.5; a tenth of 4096, mean 703:
+  // 85.3, 80.2, 63.2; one of 32768, mean 529: 150, 499, 137; uniform to 32768 1597,
+  // 1238, 1225; uniform to 4096 174.9, 171.3, 171.3 (split 175.9).  Equal lengths
+  // of 12000, [96], pay: 766, 697, 705.
+  if (MODE == kModePaged && p.B * per_seq >= kUnsplitUnits && longest <= min(kMaxChunk, 2 * round + kSplitCost))
+    want = longest;
   RaggedItem it;
   it.chunk = max(1, (want + kChunkQuantum - 1) / kChunkQuantum) * kChunkQuantum;
   const float inv = 1.0f / static_cast<float>(it.chunk);

@@ -51,7 +51,11 @@ def test_continuous_batching_planned(fa, kind, b, hq, hkv, n, d):
 @pytest.mark.parametrize("kind", ["uniform", "equal", "edges", "one_long", "overrun"])
 @pytest.mark.parametrize("b,hq,hkv,n,d", [(64, 16, 4, 1100, 64), (65, 8, 4, 900, 128), (129, 8, 2, 1300, 64),
                                           (16, 32, 8, 2500, 64), (512, 2, 1, 600, 64), (513, 2, 1, 600, 64),
-                                          (256, 4, 2, 700, 64), (257, 4, 2, 700, 64)])
+                                          (256, 4, 2, 700, 64), (257, 4, 2, 700, 64),
+                                          # enough sequences to fill the CUs: split or not by the lengths
+                                          (128, 8, 8, 700, 64), (256, 8, 4, 500, 64), (512, 4, 2, 300, 64),
+                                          (800, 1, 1, 300, 64),  # (static: past the planned batches)
+                                          (100, 8, 8, 9000, 64)])
 def test_paged_planned(fa, kind, b, hq, hkv, n, d):
     g = gen(b + n + 1)
     blocks = (n + 15) // 16
@@ -79,10 +83,11 @@ def test_paged_planned(fa, kind, b, hq, hkv, n, d):
 
 
 @pytest.mark.parametrize("kind", ["uniform", "equal", "edges", "one_long"])
-@pytest.mark.parametrize("b,hq,hkv,n,d", [(128, 8, 8, 700, 64), (256, 8, 4, 500, 64)])
+@pytest.mark.parametrize("b,hq,hkv,n,d", [(128, 8, 8, 700, 64), (256, 8, 4, 500, 64), (100, 8, 8, 21000, 64)])
 def test_paged_planned_equals_single_sequences(fa, kind, b, hq, hkv, n, d):
     """Every sequence of a batch that fills the CUs against a call with that
-    sequence alone, whose splits come from its table."""
+    sequence alone, whose splits come from its table; the last size has chunks of
+    more keys than one staging of page ids holds (8192)."""
     g = gen(b + n + 2)
     blocks = (n + 15) // 16
     pages = min(b * blocks, 8192)
@@ -108,6 +113,36 @@ def test_continuous_batching_planned_equals_single_sequences(fa, kind, b, hq, hk
     one = [fa.forward_continuous_batching_fp16(q[i:i + 1], k[i:i + 1], v[i:i + 1], lens[i:i + 1], True)
            for i in range(b)]
     assert_close(out, torch.cat(one), what=f"{kind} [{b}] to {n}")
+
+
+def _call_us(call, n=20):
+    call()
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    start.record()
+    for _ in range(n):
+        call()
+    end.record()
+    end.synchronize()
+    return start.elapsed_time(end) / n * 1e3
+
+
+def test_paged_long_sequence_in_a_full_batch_is_split(fa):
+    """One long sequence among short ones must not be left to one workgroup per
+    KV head, however many sequences there are: split in the four that the
+    workspace has, the call takes an 18th of one whose sequences are all as
+    long, unsplit a 5th."""
+    b, h, n, d = 128, 8, 32768, 128
+    pages = 16384
+    g = torch.Generator(device=DEV).manual_seed(8)
+    q = torch.randn(b, 4 * h, 1, d, generator=g, device=DEV).half()
+    k, v = (torch.randn(pages, h, 16, d, generator=g, device=DEV).half() for _ in range(2))
+    table = torch.randint(0, pages, (b, n // 16), generator=g, device=DEV, dtype=torch.int32)
+    lens = torch.full((b,), n, dtype=torch.int32, device=DEV)
+    call = lambda: fa.forward_paged_decode_gqa_fp16(q, k, v, table, lens, n // 16)
+    every = _call_us(call)
+    lens.fill_(100)
+    lens[b // 2] = n
+    assert 8 * _call_us(call) < every
 
 
 def test_planned_calls_replay_with_other_lengths(fa):
