@@ -315,9 +315,21 @@ struct TileRing {
     }
   }
 
+  // The thread index; opaque to the compiler in fp32's split blocks at DP = 64, so
+  // that the register path's addresses are formed anew for each tile (a few VALU
+  // instructions) and not kept in registers: the key-major kernel has none left
+  // there (5 went to scratch: causal [1,8,2048,64] backward 371 -> 363 us without).
+  // Unsplit blocks have them, and pay ([4,16,2048,64] 1053 -> 1096).
+  __device__ __forceinline__ int thread_now() const {
+    int t = tid;
+    if constexpr (sizeof(T) == 4 && DP == 64 && SR > kRows) asm volatile("" : "+v"(t));
+    return t;
+  }
+
   // Register path: load rows [r0, r0 + SR) (zero past `rows`) into registers ...
   __device__ __forceinline__ void load(const T* pa, const T* pb, const float* va, const float* vb, int r0, int rows,
                                        int d) {
+    const int tid = thread_now();
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i) {
       const int c = tid + i * kThreads;
@@ -343,6 +355,7 @@ struct TileRing {
   __device__ __forceinline__ void store(int stage) const {
     lds_ptr<T> ta = tile_a(stage);
     lds_ptr<T> tb = tile_b(stage);
+    const int tid = thread_now();
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i) {
       const int c = tid + i * kThreads;

@@ -52,7 +52,8 @@ def scratch():
     return {k[".name"]: k[".private_segment_fixed_size"] for elf in code_objects(blob) for k in kernels(elf)}
 
 
-@pytest.mark.parametrize("kernel", ["verify_kernel", "evict_kernel", "decode_splitkv_kernel"])
+@pytest.mark.parametrize("kernel", ["verify_kernel", "evict_kernel", "decode_splitkv_kernel", "query_major_kernel",
+                                    "dkdv_kernel"])
 def test_no_scratch(scratch, kernel):
     found = {n: s for n, s in scratch.items() if kernel in n}
     assert found
