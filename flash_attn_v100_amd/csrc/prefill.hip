@@ -737,7 +737,7 @@ static int dispatch_prefill(const char* fn, int D, bool vec, int rows_max, Prefi
   if (D <= 128 && whole <= kSplit4MaxBlocks) ks = 4;
   else if (whole <= kSplit2MaxBlocks) ks = rows_max > 64 && (D <= 128 || whole <= 128 || rows_max > 512) ? 2 : 1;
   else if (whole <= 2 * kSplit2MaxBlocks && D <= 128 && p.causal && rows_max > 1024) ks = 2;
-  p.qtiles = ceil_div(rows_max, prefill_bq(D) / ks);
+  p.qtiles = ceil_div(rows_max, ks > 1 ? 32 * kPreWaves / ks : prefill_bq(D));  // (split blocks are of 32 rows)
 #if FA_PRE_ORDER == 0
   const long long main_blocks = static_cast<long long>(p.qtiles) * p.H_Q * p.B;
 #else
