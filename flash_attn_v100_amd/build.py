@@ -71,8 +71,8 @@ def build_library(verbose: bool = True) -> str:
     """Compile the HIP kernels and the C ABI into libflash_attn_mi355x.so.
 
     ``FA_EXTRA_HIPFLAGS`` (environment, space-separated) is appended to every
-    kernel compile: it is how measurement builds switch on the tuning and
-    ablation macros the kernel sources document (e.g. ``-DFA_ABL_NOCOPY``).
+    kernel compile: it is how measurement builds set the tuning macros that
+    the kernel sources document (e.g. ``-DFA_PRE_W128=4``).
     The shipped build leaves it unset."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     objs = []

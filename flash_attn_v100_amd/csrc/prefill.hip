@@ -81,14 +81,6 @@ struct PrefillParams {
 
 // Tile shape per padded head dim.  The FA_PRE_* macros are tuning hooks for
 // building variants; the defaults are the shipped configuration.
-//
-// Ablation hooks (FA_ABL_*, off by default) remove one part of the tile loop
-// so that a timed run shows what that part costs; such a build computes wrong
-// results and is only ever timed:
-//   FA_ABL_NOCOPY   no tile copies after the first NS - 1 (the waits return at once)
-//   FA_ABL_HOTCOPY  every copy reads the sequence's first tile (always cache-resident)
-//   FA_ABL_NOQK     no QK^T MFMAs (and no K fragment reads)
-//   FA_ABL_NOPV     no P V MFMAs
 #ifndef FA_PRE_RB64
 #define FA_PRE_RB64 1
 #endif
@@ -300,14 +292,7 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
     cp_off[i] = static_cast<unsigned>((cp_row[i] * stride + cp_col[i]) * sizeof(half_t));
   }
   auto issue = [&](int t) {
-#ifdef FA_ABL_NOCOPY
-    if (t >= NS - 1) return;
-#endif
-#ifdef FA_ABL_HOTCOPY
-    const int kt = 0;
-#else
     const int kt = t * kBK;
-#endif
     const unsigned sk = lds_base + (t % NS) * kStageBytes;
     const half_t* kb = kp + static_cast<size_t>(kt) * stride;
     const half_t* vb = vp + static_cast<size_t>(kt) * stride;
@@ -421,11 +406,7 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
         const half8_t a = *lds_at<half8_t>((kaddr ^ (32 * kk)) + blk * 32 * DP * 2);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-#ifdef FA_ABL_NOQK
-          if (kk == 0) sacc[blk][rb][0] += static_cast<float>(a[0]);
-#else
           sacc[blk][rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[rb][kk], sacc[blk][rb], 0, 0, 0);
-#endif
         }
       }
     }
@@ -518,11 +499,7 @@ __attribute__((amdgpu_waves_per_eu(PrefillShape<DP, WIDE, KS, DC>::WAVES_PER_SIM
         const half8_t a = kEarlyReads ? vf[kEarlyReads ? db : 0][i & 1] : v_frag(db, i);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-#ifdef FA_ABL_NOPV
-          oacc[db][rb][i] += static_cast<float>(a[0]) + static_cast<float>(pf[rb][i][0]);
-#else
           oacc[db][rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pf[rb][i], oacc[db][rb], 0, 0, 0);
-#endif
         }
       }
     }
