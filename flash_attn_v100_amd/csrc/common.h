@@ -125,6 +125,37 @@ __device__ __forceinline__ void wait_vmem_stores() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
+// x of the lane that DPP control CTRL names, 0 where it names none (gfx9 row
+// shifts and row broadcasts; ROWS masks the rows of 16 lanes that take part).
+constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
+constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+template <int CTRL, int ROWS = 0xF, typename T>
+__device__ __forceinline__ T dpp_from(T x) {
+  static_assert(sizeof(T) == 4, "one register");
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xF, false));
+}
+
+// Inclusive scans over a wave.
+template <typename T>
+__device__ __forceinline__ T wave_scan_add(T x) {
+  x += dpp_from<kRowShr1>(x);
+  x += dpp_from<kRowShr2>(x);
+  x += dpp_from<kRowShr4>(x);
+  x += dpp_from<kRowShr8>(x);
+  x += dpp_from<kRowBcast15, 0xA>(x);
+  x += dpp_from<kRowBcast31, 0xC>(x);
+  return x;
+}
+__device__ __forceinline__ int wave_scan_max(int x) {  // x >= 0
+  x = max(x, dpp_from<kRowShr1>(x));
+  x = max(x, dpp_from<kRowShr2>(x));
+  x = max(x, dpp_from<kRowShr4>(x));
+  x = max(x, dpp_from<kRowShr8>(x));
+  x = max(x, dpp_from<kRowBcast15, 0xA>(x));
+  x = max(x, dpp_from<kRowBcast31, 0xC>(x));
+  return x;
+}
+
 // How a kernel reads the rows of its inputs (and writes the output's).
 enum RowMode : int {
   kRowElems = 0,   // element loads and stores: any D and alignment

@@ -159,30 +159,6 @@ __device__ __forceinline__ void preload_args(const DecodeParams& p) {
                  "s"(p.num_pages));
 }
 
-// Inclusive scans over a wave (gfx9 DPP row shifts and row broadcasts).
-template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ int dpp_shift(int x) {
-  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
-}
-__device__ __forceinline__ int wave_scan_add(int x) {
-  x += dpp_shift<0x111>(x);
-  x += dpp_shift<0x112>(x);
-  x += dpp_shift<0x114>(x);
-  x += dpp_shift<0x118>(x);
-  x += dpp_shift<0x142, 0xA>(x);
-  x += dpp_shift<0x143, 0xC>(x);
-  return x;
-}
-__device__ __forceinline__ int wave_scan_max(int x) {  // x >= 0
-  x = max(x, dpp_shift<0x111>(x));
-  x = max(x, dpp_shift<0x112>(x));
-  x = max(x, dpp_shift<0x114>(x));
-  x = max(x, dpp_shift<0x118>(x));
-  x = max(x, dpp_shift<0x142, 0xA>(x));
-  x = max(x, dpp_shift<0x143, 0xC>(x));
-  return x;
-}
-
 template <int MODE>
 __device__ __forceinline__ int seq_len_of(const DecodeParams& p, int b) {
   if constexpr (MODE == kModeCB) {
@@ -478,7 +454,8 @@ __device__ __forceinline__ RaggedItem ragged_item(const DecodeParams& p, int S) 
 
 template <int DP, int GB, int MODE, int ROWS, bool LDSK>
 // Registers are the compiler's choice under the 256-thread bound (94-256
-// VGPRs across the instantiations, none spilling); asking for four waves per
+// VGPRs, and AGPRs beside them where element rows meet 16 heads at D > 64;
+// nothing goes to scratch); asking for four waves per
 // SIMD made the INT8 KV cache spill (128 registers) and run 14 % slower.
 __global__ __launch_bounds__(kDecThreads) void decode_splitkv_kernel(
     DecodeParams p) {

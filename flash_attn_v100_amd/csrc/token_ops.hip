@@ -299,44 +299,16 @@ __device__ __forceinline__ uint32_t advance(uint32_t n, Inc a) {
   return n + ((n & 1u) ? d1 : d0);
 }
 
-// x of the lane that DPP control CTRL names, 0 (no increment) where it names none
-template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ uint32_t dpp_from(uint32_t x) {
-  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, ROWS, 0xF, false));
-}
 template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ void scan_step(Inc& x) {
   const Inc below = {dpp_from<CTRL, ROWS>(x.d0), dpp_from<CTRL, ROWS>(x.d1)};
   x = then(below, x);
 }
-constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
-constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
-
-template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ float dpp_from_f(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xF, false));
-}
-
-// Inclusive scans over the wave.
-__device__ __forceinline__ float scan_sum(float x) {
-  x += dpp_from_f<kRowShr1>(x);
-  x += dpp_from_f<kRowShr2>(x);
-  x += dpp_from_f<kRowShr4>(x);
-  x += dpp_from_f<kRowShr8>(x);
-  x += dpp_from_f<kRowBcast15, 0xA>(x);
-  x += dpp_from_f<kRowBcast31, 0xC>(x);
-  return x;
-}
+// Inclusive scan over the wave.
 __device__ __forceinline__ Inc scan_inc(Inc x) {
   if (__builtin_amdgcn_ballot_w64(x.d0 != x.d1) == 0) {
     // no tie in the wave: plain increments (64 * 2^25 at most)
-    uint32_t d = x.d0;
-    d += dpp_from<kRowShr1>(d);
-    d += dpp_from<kRowShr2>(d);
-    d += dpp_from<kRowShr4>(d);
-    d += dpp_from<kRowShr8>(d);
-    d += dpp_from<kRowBcast15, 0xA>(d);
-    d += dpp_from<kRowBcast31, 0xC>(d);
+    uint32_t d = wave_scan_add(x.d0);
     d = min(d, kCap);
     return Inc{d, d};
   }
@@ -561,11 +533,11 @@ __device__ __forceinline__ int chain(const float* __restrict__ a, const float* _
       float mine = 0.0f;
 #pragma unroll
       for (int e = 0; e < kTerms; ++e) mine += t[j][e];
-      upto[j] = scan_sum(mine);
+      upto[j] = wave_scan_add(mine);
       if (lane == 63) sh.total[j * kWaves + wave] = upto[j];
     }
     __syncthreads();
-    const float chunk_end = w.s + scan_sum(sh.total[lane]);  // lane c: estimate at the end of chunk c
+    const float chunk_end = w.s + wave_scan_add(sh.total[lane]);  // lane c: estimate at the end of chunk c
     if (c0 == 0 && wave == 0) {
       __builtin_amdgcn_s_setprio(3);  // everything waits for this walk
       walk_chunk<MODE>(t[0], vw, V, r, sh.first, w);
