@@ -703,16 +703,17 @@ static int dispatch_prefill(const char* fn, int D, bool vec, int rows_max, Prefi
   //   up to 512, causal walks of more than 1024 keys (D <= 128): two
   //     ([1,32:8,1500,128] 41 -> 31, [1,32:8,2048,128] 56.4 -> 49.8, [1,16,4096,64]
   //     59.8 -> 48; but [2,32:8,1024,128] 32.2 -> 31.5, [9,8,600,128] 19.9 -> 20.4).
-  //   up to 256 at D > 128, where a split workgroup's LDS fills a CU: two past
-  //     512 keys or when each has a CU ([1,16,2048,256] 88 -> 62; [4,16,300,256]
-  //     18.1 -> 19.0; 512 blocks 185 -> 239).
+  //   up to 256 at D > 128, where a split workgroup's LDS fills a CU: two when
+  //     each has a CU, or causal past 512 keys ([1,16,2048,256] 88 -> 62; [4,16,300,256]
+  //     18.1 -> 19.0; 512 blocks 185 -> 239; full [1,16,1100,256] 53 -> 63, [1,8,4096,256]
+  //     179 -> 194).
   //   64 keys or fewer: one ([20,8,64,128] 5.3 -> 5.9; [16,8,128,128] 8.0 -> 6.8).
   //   more: one, with three or more waves per SIMD ([1,32:8,4096,128], 1024
   //     blocks, 145 -> 171 split; full [2,32:8,1024,128], 512 blocks, 42 -> 48).
   const long long whole = static_cast<long long>(ceil_div(rows_max, prefill_bq(D))) * p.H_Q * p.B;
   int ks = 1;
   if (D <= 128 && whole <= kSplit4MaxBlocks) ks = 4;
-  else if (whole <= kSplit2MaxBlocks) ks = rows_max > 64 && (D <= 128 || whole <= 128 || rows_max > 512) ? 2 : 1;
+  else if (whole <= kSplit2MaxBlocks) ks = rows_max > 64 && (D <= 128 || whole <= 128 || (p.causal && rows_max > 512)) ? 2 : 1;
   else if (whole <= 2 * kSplit2MaxBlocks && D <= 128 && p.causal && rows_max > 1024) ks = 2;
   p.qtiles = ceil_div(rows_max, ks > 1 ? 32 * kPreWaves / ks : prefill_bq(D));  // (split blocks are of 32 rows)
 #if FA_PRE_ORDER == 0
