@@ -983,6 +983,16 @@ hipStream_t backward_side_stream(hipStream_t caller, int which);
 // cannot be made.
 bool backward_events(hipEvent_t (&ev)[4]);
 
+// 128-row blocks of a call as its workgroups are dealt: eight (batch, head) units
+// at a time, one to an XCD, so a last part of eight counts whole.
+inline long long dealt_blocks(const TrainParams& p) {
+  return static_cast<long long>(p.BH < 8 ? p.BH : 8 * ceil_div(p.BH, 8)) * ceil_div(p.N, kBlockRows);
+}
+// Split blocks double the workgroups and halve each, which pays where the last
+// round of them would leave most CUs idle: 256 CUs, so the rest of the blocks by
+// 256, up to half a round.
+inline bool short_last_round(long long blocks) { return blocks % 256 > 0 && blocks % 256 <= 128; }
+
 // How a backward call runs, from the number of 128-row blocks it has (us of a
 // causal call, heavy-first single-wave blocks forked onto side streams -> the
 // rule's choice; all on one box):
@@ -1121,17 +1131,24 @@ void launch_forward_split(TrainParams p, hipStream_t st) {
   hipLaunchKernelGGL((query_major_kernel<float, DP, DP, ROWS, 0, SPLIT>), dim3(train_grid(p)), dim3(kThreads), 0, st, p);
 }
 
-// The fp32 forward splits its blocks in two at D <= 64 at every size measured
-// (causal [2,16,1000,64] 82 -> 49 us, [1,8,2048,64] 216 -> 114, [4,16,2048,64]
-// 346 -> 322; full [2,16,1024,64] 81 -> 79), and at D > 64, where a split
-// workgroup's two stages take most of a CU's LDS, only grids that leave CUs idle
-// or a lone causal workgroup on each ([2,16,512,128] 77 -> 46, [2,16,1000,128]
-// 151 -> 96-119; full [2,16,1024,128] 155 unsplit, 171 split).
+// The fp32 forward splits its blocks in two (us, whole -> split):
+//  * D <= 64, causal, D <= 32 or fewer than 8 heads: always ([2,16,1000,64] 78 -> 49,
+//    [1,8,2048,64] 201 -> 111, [8,16,1000] 197 -> 177; full [2,16,1700,32] 130 -> 124,
+//    [1,4,6000,64] 442 -> 423).
+//  * D <= 64, full: with a short last round, up to three ([1,16,2500] 327 -> 279,
+//    [4,16,640] 89 -> 78, [1,40,1700] 329 -> 312; not [4,16,1000], 512 blocks, 140 -> 157,
+//    [1,40,1300], 440, 174 -> 195, [4,16,1300], 704, 253 -> 289, [1,40,400], 160, 35 -> 37).
+//  * D > 64, where a split workgroup's two stages take most of a CU's LDS: only
+//    grids that leave CUs idle or a lone causal workgroup of more than two blocks'
+//    walk on each ([2,16,512,128] 73 -> 44, [2,16,1000,128] 142 -> 114; full
+//    [2,16,1000,128] 145 -> 163, [1,12,1150] 163 -> 175; causal [8,16,256,128] 42.1 -> 45.6).
 template <int DP, int ROWS>
 void launch_forward_dp(const TrainParams& p, hipStream_t st) {
   if constexpr (ROWS != kRowElems) {
-    const long long blocks = static_cast<long long>(p.BH) * ceil_div(p.N, kBlockRows);
-    if (DP <= 64 || blocks <= (p.causal ? 256 : 128)) {
+    const long long dealt = dealt_blocks(p), blocks = static_cast<long long>(p.BH) * ceil_div(p.N, kBlockRows);
+    const bool split = DP <= 64 ? p.causal || DP <= 32 || p.BH < 8 || (dealt <= 768 && short_last_round(dealt))
+                                : (p.causal ? blocks <= (p.N > 256 ? 256 : 128) : dealt <= 128);
+    if (split) {
       launch_forward_split<DP, ROWS, 2>(p, st);
       return;
     }
@@ -1146,7 +1163,8 @@ inline void launch_forward_fp32(const TrainParams& p, bool aligned, hipStream_t 
     if (D <= 32) launch_forward_dp<32, kRowElems>(p, st);
     else if (D <= 64) launch_forward_dp<64, kRowElems>(p, st);
     else launch_forward_dp<128, kRowElems>(p, st);
-  } else if (D <= 32) launch_forward_dp<32, kRowChunks>(p, st);
+  } else if (D == 32) launch_forward_dp<32, kRowFull>(p, st);
+  else if (D < 32) launch_forward_dp<32, kRowChunks>(p, st);
   else if (D == 64) launch_forward_dp<64, kRowFull>(p, st);
   else if (D < 64) launch_forward_dp<64, kRowChunks>(p, st);
   else if (D <= 96) launch_forward_dp<96, kRowChunks>(p, st);
