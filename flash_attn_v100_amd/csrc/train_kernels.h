@@ -993,19 +993,43 @@ inline long long dealt_blocks(const TrainParams& p) {
 // 256, up to half a round.
 inline bool short_last_round(long long blocks) { return blocks % 256 > 0 && blocks % 256 <= 128; }
 
-// How a backward call runs, from the number of 128-row blocks it has (us of a
-// causal call, heavy-first single-wave blocks forked onto side streams -> the
-// rule's choice; all on one box):
-//  * fp16, up to 512 blocks: split in two, in order on the caller's stream (the
-//    fork and its events cost the host 30 us): [1,8,128,128] 61 -> 32,
-//    [2,16,512,128] 61 -> 43, [1,8,2048,128] 160 -> 109, [2,16,1000,64] 66 -> 47.
-//  * fp16, more: unsplit; D > 64 forked, dQ as a snake ([4,16,2048,128] 316, heavy
-//    first 320, in order 336, split 370), D <= 64 in order ([4,16,2048,64] 187 -> 167).
-//  * fp32 D <= 64: in order; split up to 512 blocks ([2,16,1000,64] 259 -> 183,
-//    [1,8,2048,64] 582 -> 381; [4,16,2048,64] 1193 -> 1054 unsplit).
+// How a backward call runs, from its 128-row blocks, their walk and the mask (us,
+// heavy-first whole blocks forked onto side streams -> the rule's choice, each
+// in a process of its own on one box; "split" is two waves a block, in order on the
+// caller's stream unless forked: the fork and its events cost the host 30 us).
+//  * fp16 D > 64
+//    - past 2048 rows, full on at most 192 blocks or causal of fewer than 8 heads
+//      (which no order balances) on at most 256: split and forked, so that the passes
+//      share idle CUs (causal [1,4,6000,128] 265 -> 246, in order 319; full [1,8,2500]
+//      159 -> 162, 182).
+//    - up to 512 blocks: split (causal [1,8,2048,128] 148 -> 107, [2,16,1000] 84 -> 71;
+//      full [1,16,1000] 83 -> 65), but
+//      full past 384: whole in order ([1,16,3300] 406 -> 407, split 463; [4,16,1000]
+//      179 -> 169, 194); full past 256 and 512 rows: whole and forked ([1,16,2500]
+//      259, split 299; [4,16,400] 69 -> 54 split);
+//      causal of more than 16 heads and 1024 rows past 432, of more than 32 (a last,
+//      part group of units an XCD) past 352: as below ([2,16,2048] 182 -> 179, split
+//      193; [3,12,1300] 139, 162; but [2,16,1300] 107 -> 100 split, [1,16,4096] 420 -> 365).
+//      Only rows wider than 96 columns: narrower, [3,12,1150,96] full 149 split, 158.
+//    - more: whole and forked, dQ as a snake ([4,16,2048,128] 316, heavy first 320,
+//      in order 336, split 370).
+//  * fp16 D <= 64: in order, up to 512 blocks split ([1,16,2048,64] 96 -> 64); past
+//    them whole ([4,16,2048,64] 187 -> 172), but full calls of a short last round split
+//    up to 1280 ([1,40,3300] 476 -> 480, whole 495; [4,16,2300] 365 -> 368, 381; not
+//    [4,16,1300], 704 blocks, 153 -> 141 whole, 150), longer ones forked up to 2048
+//    ([4,16,2800] 511, whole or split 528; [8,16,1900] 492, 513).
+//  * fp32 D <= 64: in order, but causal past 2048 rows of fewer than 8 heads, up to 256
+//    blocks, as fp16's ([1,4,6000,64] 1353 -> 985, in order 1195); split up to 512
+//    blocks ([1,16,2048,64] 598 -> 366) and, past them, causal ([8,16,1000] 670 -> 584,
+//    whole 718; [4,16,1300] 580 -> 501, 523; not [8,16,640], five blocks a head, 319 ->
+//    266 whole, 276) or full with a short last round ([1,40,1700] 1064 -> 1012, 1177;
+//    not [8,16,1000] 1045 -> 942 whole, 978).
 //  * fp32 D > 64: forked; up to 128 blocks split and dQ's blocks light first,
-//    against dK/dV's heavy first on the same CUs ([1,8,2048,128] 1110 -> 870,
-//    [2,16,512,128] 181 -> 121; [2,16,1000,128] 349 either way).
+//    against dK/dV's heavy first on the same CUs ([1,8,2048,128] 1107 -> 862,
+//    [2,16,512,128] 183 -> 125).  With 20-23 or 27-31 split blocks of a kernel on an
+//    XCD's 32 CUs, or more than fit it, that pairing misses and both run as snakes
+//    ([1,8,1344] 462 -> 431, light first 526; [1,8,1856] 847 -> 680, 978; [1,12,1184] 397
+//    -> 401, 458; but [1,8,1536], 24 blocks, 679 -> 515, snakes 600).  More: whole.
 struct BackwardPlan {
   int split;
   bool fork;
@@ -1013,12 +1037,36 @@ struct BackwardPlan {
 };
 template <typename T, int DP>
 BackwardPlan backward_plan(const TrainParams& p) {
-  const long long blocks = static_cast<long long>(p.BH) * ceil_div(p.N, kBlockRows);
-  if (sizeof(T) == 4 && DP > 64)
-    return blocks <= 128 ? BackwardPlan{2, true, kLightFirst, kHeavyFirst} : BackwardPlan{1, true, kHeavyFirst, kHeavyFirst};
-  if (blocks <= 512) return BackwardPlan{2, false, kSnake, kSnake};
-  if (sizeof(T) == 4) return BackwardPlan{1, false, kHeavyFirst, kHeavyFirst};
-  if (DP > 64) return BackwardPlan{1, true, kSnake, kHeavyFirst};
+  constexpr BackwardPlan kSplit = {2, false, kSnake, kSnake}, kSplitForked = {2, true, kSnake, kHeavyFirst};
+  constexpr BackwardPlan kForked = {1, true, kHeavyFirst, kHeavyFirst};
+  const bool causal = p.causal != 0;
+  if (sizeof(T) == 4 && DP > 64) {
+    if (static_cast<long long>(p.BH) * ceil_div(p.N, kBlockRows) > 128) return kForked;
+    const int n = ceil_div(p.BH, 8) * ceil_div(p.N, kBlockRows / 2);  // each kernel's split blocks on an XCD
+    const bool miss = causal && p.N > 512 && (n > 32 || (p.BH % 8 == 0 && ((n >= 20 && n < 24) || (n >= 27 && n < 32))));
+    return miss ? BackwardPlan{2, true, kSnake, kSnake} : BackwardPlan{2, true, kLightFirst, kHeavyFirst};
+  }
+  const long long blocks = dealt_blocks(p);
+  const bool few_long = p.N > 2048 && p.BH < 8 && causal;
+  if (sizeof(T) == 4) {
+    if (few_long && blocks <= 256) return kSplitForked;
+    if (blocks <= 512 || (causal ? blocks > 768 || p.N > 768 : blocks <= 1024 && short_last_round(blocks))) return kSplit;
+    return BackwardPlan{1, false, kHeavyFirst, kHeavyFirst};
+  }
+  if (DP > 64 && p.D <= 96) return blocks <= 512 ? kSplit : BackwardPlan{1, true, kSnake, kHeavyFirst};
+  if (DP > 64) {
+    if ((few_long && blocks <= 256) || (p.N > 2048 && !causal && blocks <= 192)) return kSplitForked;
+    if (blocks > 512 || (causal && p.N > 1024 && p.BH > 16 && blocks > (p.BH > 32 ? 352 : 432)))
+      return BackwardPlan{1, true, kSnake, kHeavyFirst};
+    if (!causal && blocks > 384) return BackwardPlan{1, false, kSnake, kSnake};
+    if (!causal && blocks > 256 && p.N > 512) return kForked;
+    return kSplit;
+  }
+  if (blocks <= 512) return kSplit;
+  if (!causal && short_last_round(blocks)) {
+    if (blocks <= 1280) return kSplit;
+    if (blocks <= 2048 && p.N > 1024) return kForked;
+  }
   return BackwardPlan{1, false, kSnake, kSnake};
 }
 
@@ -1106,7 +1154,8 @@ void launch_backward(const TrainParams& p, bool aligned, hipStream_t st) {
       if (D <= 32) launch_backward_dp<T, 32, 32, kRowElems>(p, st);
       else if (D <= 64) launch_backward_dp<T, 64, 64, kRowElems>(p, st);
       else launch_backward_dp<T, 128, 128, kRowElems>(p, st);
-    } else if (D <= 32) launch_backward_dp<T, 32, 32, kRowChunks>(p, st);
+    } else if (D == 32) launch_backward_dp<T, 32, 32, kRowFull>(p, st);
+    else if (D < 32) launch_backward_dp<T, 32, 32, kRowChunks>(p, st);
     else if (D == 64) launch_backward_dp<T, 64, 64, kRowFull>(p, st);
     else if (D < 64) launch_backward_dp<T, 64, 64, kRowChunks>(p, st);
     else if (D <= 96) launch_backward_dp<T, 96, 96, kRowChunks>(p, st);

@@ -90,9 +90,9 @@ size_t fa_backward_workspace_size(int B, int H, int N);
  * 1 <= D <= 128.  Two or three launches on `stream` (dQ with the row
  * statistic delta = rowsum(dout * out) into the workspace, then dK/dV, as one
  * pass or as a dV and a dK pass); deterministic (no atomics).  The workspace needs no initialisation.
- * Large calls (fp16 at D > 64 past 512 blocks of 128 rows), fp32 ones at
- * D > 64 and those whose rows are not whole aligned groups of 8 elements
- * take delta, outside graph capture, from a short kernel of its own and run the
+ * Some long or large calls, fp32 ones at D > 64 and those whose rows are not
+ * whole aligned groups of 8 elements take delta, outside graph capture, from a
+ * short kernel of its own and run the
  * dK/dV work (fp16: the dV and the dK pass) on library-owned
  * side streams of the device (non-blocking, default priority) concurrently
  * with the dQ kernel, forked

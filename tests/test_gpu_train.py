@@ -255,3 +255,53 @@ def test_backward_on_several_caller_streams(fa, dtype):
     for r, x in zip(ref, got):
         for a, e in zip(x, r):
             assert torch.equal(a, e)
+
+
+F16, F32 = torch.float16, torch.float32
+
+
+@pytest.mark.parametrize("dtype,b,h,n,d,causal", [
+    # fp16, D > 96: split and forked (long, few blocks), whole in order, whole and forked (two thresholds)
+    (F16, 1, 2, 2100, 128, True), (F16, 1, 2, 2100, 128, False), (F16, 40, 10, 100, 128, False),
+    (F16, 5, 11, 520, 128, False), (F16, 1, 40, 1030, 128, True), (F16, 1, 17, 2060, 104, True),
+    # fp16, D <= 64 past 512 blocks, full: a short last round split, or forked; a full one whole
+    (F16, 52, 10, 100, 64, False), (F16, 24, 6, 1030, 64, False), (F16, 70, 10, 100, 64, False),
+    # fp32, D <= 64: split and forked; past 512 blocks split, whole
+    (F32, 1, 2, 2100, 64, True), (F32, 80, 10, 100, 64, True), (F32, 60, 10, 100, 48, True),
+    (F32, 52, 10, 100, 64, False), (F32, 70, 10, 100, 32, False),
+    # fp32, D > 64, up to 128 blocks: both as snakes, or light against heavy first; the
+    # forward with and without split blocks
+    (F32, 1, 8, 1300, 128, True), (F32, 1, 12, 1184, 96, True), (F32, 1, 8, 1100, 128, True),
+    (F32, 10, 16, 200, 128, True), (F32, 10, 16, 300, 72, True), (F32, 1, 12, 1150, 128, False)])
+def test_training_plans(fa, dtype, b, h, n, d, causal):
+    """Every way a call can be split, ordered and forked: first, middle and last
+    head against the oracle, and the same bits from a second call and from replays
+    of a captured one, which stays on its stream."""
+    g = gen(b * h + n + d)
+    q, k, v, do = (randn(g, b, h, n, d, dtype=dtype) for _ in range(4))
+    qc, kc, vc, dc = cuda(q, k, v, do)
+    fwd = fa.forward_fp16_with_lse if dtype == F16 else fa.forward_with_lse
+    out, lse = fwd(qc, kc, vc, causal)
+    grads = fa.backward(dc, qc, kc, vc, out, lse, causal)
+    for i in sorted({0, b * h // 2, b * h - 1}):
+        one = lambda t: t.reshape(b * h, n, -1)[i].reshape(1, 1, n, -1).cpu()
+        lse_i = lse.reshape(b * h, n)[i].reshape(1, 1, n).cpu()
+        ro, rl = A.prefill_lse(one(q), one(k), one(v), causal, compute_dtype=F64)
+        tol = dict(atol=2e-3, rtol=1e-2) if dtype == F16 else dict(atol=2e-4, rtol=2e-4)
+        assert_close(one(out), ro, what=f"out, head {i}", **tol)
+        assert_close(lse_i, rl, atol=tol["atol"], rtol=tol["atol"], what=f"lse, head {i}")
+        ref = A.backward(one(do), one(q), one(k), one(v), one(out), lse_i, causal)
+        _check_grads([one(t) for t in grads], ref, dtype == F16, f"head {i}")
+    for a, r in zip(fa.backward(dc, qc, kc, vc, out, lse, causal), grads):
+        assert torch.equal(a, r)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = fa.backward(dc, qc, kc, vc, out, lse, causal)
+    for _ in range(3):
+        for t in captured:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, r in zip(captured, grads):
+            assert torch.equal(a, r)
