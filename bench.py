@@ -386,7 +386,8 @@ def cfg9_speculative_verify(fa, torch, steps, warmup):
     """speculative_verify: B=16 rows, K=4 draft tokens, vocabulary 32000 (the
     reference test's large case).  Independent random target/draft
     distributions, so most rows reject early and run the full residual scans.
-    Latency-bound: each sampled index comes from a serial fp32 running sum."""
+    Latency-bound: each sampled index has the value of a serial fp32 running
+    sum, which parallel scans compute bit for bit."""
     B, K, V = 16, 4, 32000
     gg = torch.Generator(device="cuda").manual_seed(90)
     tp = torch.softmax(torch.randn(B, K + 1, V, generator=gg, device="cuda"), -1)
@@ -397,7 +398,7 @@ def cfg9_speculative_verify(fa, torch, steps, warmup):
     acc, _ = fa.speculative_verify(tp, dp, tok, rv, K)
     return dict(workload="speculative_verify B=16 K=4 vocab=32000", ms=ms, us_per_call=ms * 1e3,
                 rows_per_s=B / (ms * 1e-3), mean_accepted=float(acc.float().mean().item()),
-                bound="serial fp32 running sums (latency)"), (tp[:2].cpu(), dp[:2].cpu(), tok[:2].cpu(), rv[:2].cpu(), K)
+                bound="assembly of exact fp32 running sums (latency)"), (tp[:2].cpu(), dp[:2].cpu(), tok[:2].cpu(), rv[:2].cpu(), K)
 
 
 # ----------------------------------------------------------------------------- ceilings

@@ -287,7 +287,7 @@ __device__ __forceinline__ int counter_index(int slot) {
 // length, longest first.
 // Uniform lengths, D = 128, 32:8 heads (us, static -> planned): continuous
 // batching [64] to 8192 keys 171.7 -> 164.0, [128] to 4096 256 -> 191, [32] to 2048
-// 32.3 -> 28.9, [128] to 256 29.5 -> 19.8; paged [128] to 4096 186.6 -> 184.8
+// 32.3 -> 28.9, [128] to 257 28.6 -> 19.5; paged [128] to 4096 186.6 -> 184.8
 // (split in 2048 192), [64] to 8192 212 -> 189, [16] to 2048 26.1 -> 14.1, [64] to
 // 1024 34 -> 26.7.  One round against 2048 workgroups: paged [32] to 2048 28.9,
 // 31.1; continuous batching [100,32:4] to 1500 26.0, 31.3, but [64] to 8192 209,
@@ -1555,9 +1555,9 @@ static int run_decode(const char* fn, DecodeParams p, int max_len, void* ws, siz
   const long long units = static_cast<long long>(p.B) * p.H_KV * pl.num_hg;
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Continuous batching that no plan would split (one workgroup per unit either
-  // way) skips the planning: uniform lengths, 32:8 heads, D = 128, to 256 keys,
-  // planned -> static: [128] 20.9 -> 17.4 us, [256] 45 -> 32 (paged gains from the
-  // order even then: [128] 21.2, in sequence order with ranks in LDS 26.5).
+  // way) skips the planning: uniform lengths to 256 keys, 32:8 heads, D = 128, [128]
+  // 20.9 -> 17.4 us (paged gains from the order even then: [128] 21.2, in sequence
+  // order with ranks in LDS 26.5).
   const bool plannable = MODE == kModePaged || pl.splits > 1;
   if (!kFixed && plannable && units * pl.splits > kStaticMaxBlocks && p.B <= kPlanMaxSeqs &&
       units <= static_cast<long long>(kCounterSlots)) {

@@ -264,10 +264,12 @@ def test_continuous_batching(fa, causal, b, hq, hkv, d, max_n, cls):
 
 
 @pytest.mark.parametrize("b,cls", [
-    (12, [40, 7, 40, 40, 0, 7, 90, 40, 7, 90, 3, 40]),   # ties: the longest-first order must stay a bijection
-    (600, None),                                          # more sequences than the longest-first limit (natural order)
+    (12, [40, 7, 40, 40, 0, 7, 90, 40, 7, 90, 3, 40]),
+    (600, None),
 ])
 def test_continuous_batching_ordering(fa, b, cls):
+    """Lengths in no order, with ties, in calls that no split plan serves: a
+    workgroup per sequence and KV head, in index order."""
     g = gen(12)
     hq, hkv, d, max_n = 4, 2, 64, 96
     if cls is None:
@@ -375,12 +377,14 @@ def test_paged_decode_random_tables(fa, hq, hkv, d):
 
 
 @pytest.mark.parametrize("b,sls", [
-    (12, [40, 7, 40, 40, 1, 7, 90, 40, 7, 90, 3, 40]),   # longest first with ties: the order must stay a bijection
-    (600, None),                                          # more sequences than the longest-first limit (natural order)
+    (12, [40, 7, 40, 40, 1, 7, 90, 40, 7, 90, 3, 40]),   # too few workgroups to plan: index order
+    (320, None),                                          # planned: classes of length, longest first, with ties
+    (600, None),                                          # more sequences than are planned: index order
 ])
 def test_paged_decode_ordering(fa, b, sls):
-    """Paged decode serves sequences longest first (ties by index) for up to
-    512 sequences and in index order beyond; every row against the oracle."""
+    """Paged decode deals planned batches (past 600 workgroups, up to 512
+    sequences) by length, a one-to-one map whatever the ties, and others in index
+    order; every row against the oracle."""
     g = gen(13)
     hq, hkv, d, mnb = 4, 2, 64, 6
     if sls is None:
