@@ -503,12 +503,13 @@ __device__ __forceinline__ Terms make_terms(const Terms& a, const Terms& b, floa
 //  kPrefix:   cs += a; hit when r < cs.
 //  kBonus:    cs += a; hit when cs >= r.
 // Returns the reference's token: the first hit past index 0 (there, a hit at
-// index 0 is replaced by the next one), 0 without one.  Every wave takes the same path through the
-// barriers: what decides it is read from LDS after one.  Indices are unsigned:
-// the last group's ends pass 2^31 when V is within a group of it.
+// index 0 is replaced by the next one), 0 without one.  Every wave takes the
+// same path through the barriers: what decides it is read from LDS after one.
+// Indices are unsigned: the last group's ends pass 2^31 when V is within a
+// group of it.
 template <int MODE>
-__device__ __forceinline__ int chain(const float* __restrict__ a, const float* __restrict__ b, uint32_t V, float Z, float r, float* sum,
-                     Shared& sh) {
+__device__ __forceinline__ int chain(const float* __restrict__ a, const float* __restrict__ b, uint32_t V, float Z,
+                                     float r, float* sum, Shared& sh) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr bool kDiff = MODE == kZ || MODE == kResidual;

@@ -1,8 +1,8 @@
 """Continuous batching and paged decode with the splits planned from the lengths
-on the device: every sequence against the CPU oracle, at batch sizes on both
-sides of the planner's register blocks (64, 128, 256 and 512 sequences) and past it,
-with empty and negative lengths, lengths on and next to chunk boundaries, all
-equal, and one long sequence among short ones."""
+on the device: sequences against the CPU oracle, and all of them against calls with
+one alone, at batch sizes on both sides of the planner's register blocks (64, 128, 256
+and 512 sequences) and past it, with empty and negative lengths, lengths on and next
+to chunk boundaries, all equal, and one long sequence among short ones."""
 import pytest
 import torch
 
